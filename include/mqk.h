@@ -318,9 +318,12 @@ int mqk_fused_qkv_rope_paged_w4a16(const mqk_bf16* x, const int32_t* qw_q, const
  * Input RMSNorm (in_gamma != NULL): the projection input is
  * in_gamma * bf16(x_fp32 * rsqrt(mean(x^2) + in_eps)), rounded to bf16 -- the
  * decoder layer's input_layernorm (mini_qwen/model/layers/rms_norm.py:11-18,
- * applied at mini_qwen/model/qwen3.py:58-59) computed inside the op, so the
- * normalised activations never go to HBM.  The per-token scale is computed by a
- * pre-pass into the workspace: size it with mqk_fused_qkv_rope_ex_workspace_size.
+ * applied at mini_qwen/model/qwen3.py:58-59) computed inside the op: a pre-pass
+ * writes the normalised rows to the workspace, sized with
+ * mqk_fused_qkv_rope_ex_workspace_size.  In a workspace with room only for the
+ * plain size (at least the counters) and T floats, the pre-pass writes the
+ * per-token scales and the projection normalises what it stages: slower, the same
+ * values.
  *
  * kv != NULL: the paged KV-cache write of mqk_fused_qkv_rope_paged_* (in
  * varlen mode kv_seq / kv_pos may be NULL: the sequence and position above).
@@ -334,8 +337,9 @@ typedef struct mqk_fused_ext {
   const mqk_paged_kv* kv;       /* paged KV cache, or NULL */
 } mqk_fused_ext;
 
-/* Workspace bytes needed by the _ex entry points (the plain size plus the
- * input-norm scales when ext->in_gamma is set). */
+/* Workspace bytes of the _ex entry points (the plain size, plus the normalised rows
+ * when ext->in_gamma is set, or the per-token scales where the rows would exceed
+ * 256 MiB). */
 size_t mqk_fused_qkv_rope_ex_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden,
                                             const mqk_fused_ext* ext);
 

@@ -329,32 +329,66 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
   return pl;
 }
 
+// Pair tiles take q/k/v outputs with head_dim 128 (their epilogue splits a head in
+// 32-dim runs) and paged-cache slots below 2^31 (held in 32 bits).
+bool pair_tiles_ok(const EpilogueArgs& e) {
+  return e.qkv && e.head_dim == kHeadDim &&
+         (!e.k_cache || double(e.num_blocks) * double(e.block_size) < 2147483647.0);
+}
+
+// Workspace bytes of a plan's own region (its counters, partials and exchange
+// areas), before any normalised rows or input-norm scales.  (The decode kernel's
+// arrival counters open every workspace and must stay zero, so nothing else starts
+// before their end, whichever kernel runs the call.)
+size_t plan_region(const Plan& q, int64_t M, int n_tiles) {
+  if (q.ksplit > 0) return kDecodeCounterBytes + tile_split_part_bytes(q.v->id, M, n_tiles, q.ksplit);
+  if (q.v && is_pair_variant(q.v->id))
+    return std::max(pair_tile_workspace_bytes(q.v->id, M - q.tail, n_tiles),
+                    q.splits > 0 ? decode_workspace_bytes(n_tiles, q.splits, q.passes) : size_t(0));
+  return q.splits > 0 ? decode_workspace_bytes(n_tiles, q.splits, q.passes) : decode_counter_bytes();
+}
+
+// Bytes of normalised rows of a call with an input norm (0: too many, see
+// kNormAheadMaxBytes).
+size_t norm_ahead_bytes(int64_t M, int64_t K) {
+  const size_t n = align_up(size_t(M) * size_t(K) * 2, 256);
+  return n <= kNormAheadMaxBytes ? n : 0;
+}
+
 // Common launcher of the fused op (bf16 or int4 weights).  With an input norm
-// (p.in_gamma set, epsilon in_eps), the per-token scales go to the workspace
-// after the decode kernel's region and are computed by a pre-pass first.
+// (p.in_gamma set, epsilon in_eps), a pre-pass first writes the normalised rows to
+// the workspace after the plan's region, and the plan runs on them; a workspace
+// without that room holds the per-token scales there instead, and the projection
+// kernels normalise what they stage.
 int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& e, float in_eps,
-              void* workspace, size_t ws_bytes, hipStream_t stream) {
+              void* workspace, size_t ws_bytes, hipStream_t stream, bool allow_pair = true) {
   if (p.M == 0) return ok();
   const Topology topo = device_topology();
+  if (p.in_gamma && workspace && norm_ahead_bytes(p.M, p.K) > 0) {
+    // (pair tiles with an input norm are kept to the hidden sizes at which gamma
+    // also fits the LDS beside their ring, whichever form the workspace allows)
+    const bool pair_lds = tile_dma_lds_bytes(28) + p.K * 2 <= 160 * 1024;
+    const bool pairs = pair_lds && pair_tiles_ok(e);
+    const Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true, pairs);
+    const size_t off = align_up(plan_region(pl, p.M, p.n_tiles), 256);
+    if (ws_bytes >= off + norm_ahead_bytes(p.M, p.K)) {
+      uint16_t* xn = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
+      const int st = hip_status(launch_row_scale(p.x, p.in_gamma, p.M, p.K, in_eps, nullptr, xn, stream),
+                                "input norm pre-pass launch");
+      if (st != MQK_OK) return st;
+      p.x = xn;
+      p.in_gamma = nullptr;
+      return run_fused(int4, p, w, e, 0.f, workspace, off, stream, pair_lds);
+    }
+  }
   p.cus = topo.cus;
   p.xcds = topo.xcds;
-  // pair tiles: q/k/v outputs with head_dim 128 (their epilogue splits a head in
-  // 32-dim runs) and paged-cache slots below 2^31 (held in 32 bits)
-  const bool pair_ok = e.qkv && e.head_dim == kHeadDim &&
-                       (!e.k_cache || double(e.num_blocks) * double(e.block_size) < 2147483647.0);
+  const bool pair_ok = allow_pair && pair_tiles_ok(e);
   Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, true, pair_ok);
   if (!pl.v && pl.splits == 0)
     return fail(MQK_ERR_BAD_OPTION, "prefill_tile variant %lld cannot run this problem (%d heads%s)",
                 (long long)g_prefill_tile.load(), p.n_tiles, int4 ? ", int4 weights" : "");
-  // (the decode kernel's arrival counters open every workspace and must stay zero,
-  // so the scales never start before them, whichever kernel runs this call)
-  auto region = [&](const Plan& q) {
-    if (q.ksplit > 0) return kDecodeCounterBytes + tile_split_part_bytes(q.v->id, p.M, p.n_tiles, q.ksplit);
-    if (q.v && is_pair_variant(q.v->id))
-      return std::max(pair_tile_workspace_bytes(q.v->id, p.M - q.tail, p.n_tiles),
-                      q.splits > 0 ? decode_workspace_bytes(p.n_tiles, q.splits, q.passes) : size_t(0));
-    return q.splits > 0 ? decode_workspace_bytes(p.n_tiles, q.splits, q.passes) : decode_counter_bytes();
-  };
+  auto region = [&](const Plan& q) { return plan_region(q, p.M, p.n_tiles); };
   size_t base = region(pl);
   // bytes the plan needs: the decode (or split-tile) region, then (input norm) the per-token scales
   const size_t scale_bytes = p.in_gamma ? align_up(size_t(p.M) * sizeof(float), 256) : 0;
@@ -395,7 +429,8 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
                 workspace ? "" : " (NULL)");
   if (p.in_gamma) {
     float* scale = reinterpret_cast<float*>(static_cast<char*>(workspace) + scale_off);
-    const int st = hip_status(launch_row_scale(p.x, p.M, p.K, in_eps, scale, stream), "input norm pre-pass launch");
+    const int st = hip_status(launch_row_scale(p.x, p.in_gamma, p.M, p.K, in_eps, scale, nullptr, stream),
+                              "input norm pre-pass launch");
     if (st != MQK_OK) return st;
     p.in_scale = scale;
   }
@@ -528,8 +563,10 @@ size_t mqk_fused_qkv_rope_workspace_size_hd(int64_t T, int Hq, int Hkv, int64_t 
 size_t mqk_fused_qkv_rope_ex_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden,
                                             const mqk_fused_ext* ext) {
   size_t n = mqk_fused_qkv_rope_workspace_size(T, Hq, Hkv, hidden);
-  if (ext && ext->in_gamma && T > 0)
-    n = align_up(n > 0 ? n : decode_counter_bytes(), 256) + align_up(size_t(T) * sizeof(float), 256);
+  if (ext && ext->in_gamma && T > 0 && hidden > 0) {
+    const size_t rows = norm_ahead_bytes(T, hidden);
+    n = align_up(n > 0 ? n : decode_counter_bytes(), 256) + (rows > 0 ? rows : align_up(size_t(T) * sizeof(float), 256));
+  }
   return n;
 }
 
@@ -718,7 +755,7 @@ static int fused_bf16_any_d(const mqk_bf16* x, const mqk_bf16* w_q, const mqk_bf
       return fail(MQK_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given%s", off + size_t(T) * sizeof(float),
                   ws_bytes, workspace ? "" : " (NULL)");
     float* scale = reinterpret_cast<float*>(static_cast<char*>(workspace) + off);
-    st = hip_status(launch_row_scale(x, T, hidden, ext->in_eps, scale, hs), "input norm pre-pass launch");
+    st = hip_status(launch_row_scale(x, nullptr, T, hidden, ext->in_eps, scale, nullptr, hs), "input norm pre-pass launch");
     if (st != MQK_OK) return st;
     pn.in_scale = scale;
   }

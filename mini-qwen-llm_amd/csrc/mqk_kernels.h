@@ -149,9 +149,15 @@ hipError_t launch_tile_dma_w4(int id, const ProblemArgs& p, const WeightArgs& w,
 // LDS bytes (static) of pipelined tile variant id (10..32); 0 for other ids.
 int tile_dma_lds_bytes(int id);
 
-// Input RMSNorm pre-pass: scale[m] = rsqrt(mean(x[m, :]^2) + eps) for x [M, K] bf16.
-hipError_t launch_row_scale(const uint16_t* x, int64_t M, int64_t K, float eps, float* scale,
-                            hipStream_t stream);
+// Input RMSNorm pre-pass over x [M, K] bf16 (K <= 16384): with sc[m] =
+// rsqrt(mean(x[m, :]^2) + eps), out null: scale[m] = sc[m]; else out[m, k] =
+// bf16(gamma[k] * bf16(x[m, k] * sc[m])), the projection's input (scale unused).
+hipError_t launch_row_scale(const uint16_t* x, const uint16_t* gamma, int64_t M, int64_t K, float eps, float* scale,
+                            uint16_t* out, hipStream_t stream);
+// Most bytes of normalised rows a call keeps in its workspace; larger calls keep
+// the per-token scales only (so that one long prefill does not leave gigabytes of
+// workspace behind).
+constexpr size_t kNormAheadMaxBytes = size_t(256) << 20;
 
 int decode_splits_for(int64_t M, int64_t K, int n_tiles, int requested, int cus, int xcds);
 size_t decode_workspace_bytes(int n_tiles, int splits, int blocks = 1);

@@ -257,9 +257,14 @@ _workspaces: dict = {}
 _retired: list = []
 
 
-def workspace(device: torch.device, stream, nbytes: int):
+def workspace(device: torch.device, stream, nbytes: int, least=None):
     """The workspace of ``stream`` (a torch stream, or the raw handle of the
-    device's current stream) with at least ``nbytes`` bytes; None for 0."""
+    device's current stream) with at least ``nbytes`` bytes; None for 0.
+
+    ``least``: a function giving the bytes below which the call cannot run at all
+    (default: ``nbytes``).  During graph capture, when no buffer can be made, an
+    existing one of at least that size is returned: the call then takes the route
+    that fits it."""
     if nbytes <= 0:
         return None
     handle = stream if isinstance(stream, int) else int(stream.cuda_stream)
@@ -275,6 +280,8 @@ def workspace(device: torch.device, stream, nbytes: int):
         buf = _workspaces.get(key)
         if buf is None or buf.numel() < nbytes:
             if torch.cuda.is_current_stream_capturing():
+                if buf is not None and least is not None and buf.numel() >= least():
+                    return buf
                 raise MqkNativeError(
                     f"the mqk workspace of this stream must grow to {nbytes} bytes during HIP-graph "
                     "capture; run the op once eagerly on this stream at the largest size before capturing")
@@ -291,6 +298,8 @@ def workspace(device: torch.device, stream, nbytes: int):
 # Word of the workspace's statistics line that counts the heads the decode kernel
 # finished on its recompute path (include/mqk.h: after the 1024 arrival counters).
 _RECOMPUTE_WORD = 1024
+# The counter region that opens every workspace (kDecodeCounterBytes of csrc/mqk_kernels.h).
+_COUNTER_BYTES = 4096 + 256 + 512 * 128
 
 
 def decode_recomputes(device=None, stream=None) -> int:
@@ -355,6 +364,15 @@ def fused_workspace_bytes(T: int, H_Q: int, H_KV: int, hidden: int, D: int, ext=
                                                          ctypes.byref(ext)))
     if D not in (64, 128):
         n = max(n, int(lib.mqk_fused_qkv_rope_workspace_size_hd(T, H_Q, H_KV, hidden, D)))
+    return n
+
+
+def least_workspace_bytes(T: int, H_Q: int, H_KV: int, hidden: int, D: int, ext) -> int:
+    """The smallest workspace an _ex call runs with: without room for the rows the
+    input norm writes ahead, only for its per-token scales."""
+    n = fused_workspace_bytes(T, H_Q, H_KV, hidden, D)
+    if ext.in_gamma:
+        n = (max(n, _COUNTER_BYTES) + 255) // 256 * 256 + (4 * T + 255) // 256 * 256
     return n
 
 

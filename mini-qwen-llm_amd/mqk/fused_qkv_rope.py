@@ -386,7 +386,8 @@ def fused_qkv_rope_ex(
     lib = _native.library()
     stream = _native.stream_handle(device)
     nbytes = _native.fused_workspace_bytes(T, H_Q, H_KV, H, D, ext)
-    ws = _native.workspace(device, stream, nbytes)
+    ws = _native.workspace(device, stream, nbytes,
+                           lambda: _native.least_workspace_bytes(T, H_Q, H_KV, H, D, ext))
     status = _native.call(device, lib.mqk_fused_qkv_rope_ex_bf16,
         x.data_ptr(), w_q.data_ptr(), w_k.data_ptr(), w_v.data_ptr(),
         q_norm_w.data_ptr(), k_norm_w.data_ptr(), cos.data_ptr(), sin.data_ptr(), _native.ptr(pos),

@@ -1,0 +1,137 @@
+"""The input RMSNorm's two forms: rows normalised ahead in the workspace, and (a
+workspace without that room) in the projection kernels.
+
+Both compute bf16(gamma * bf16(x * scale)) with one scale per token and run the
+same MFMA order wherever they take the same plan, so a call at the C ABI with the
+full workspace and one with the smallest must agree: bit for bit where the launch
+is the same kernel, and within one bf16 ulp where it is not: two differently split
+fp32 sums differ by about 1e-6 of their terms, so their bf16 roundings differ by at
+most one ulp, which is up to 2^-7 of the value (at the foot of a binade); 1e-3 is
+added for values near zero.
+Sizes: one token, odd hidden chunk counts (hidden 192: 24 of 64 lanes hold chunks;
+hidden 2112: a partial fifth chunk; 16384: a row of four passes), the block and tile
+edges, and int4 weights.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+D = 128
+
+
+def _call(T, hidden, Hq, Hkv, int4, seed, device):
+    """(run(ws_bytes) -> (q, k, v), full size, smallest size)."""
+    from mqk import _native
+    lib = _native.library()
+    g = torch.Generator(device=device).manual_seed(seed)
+    x = (3 * torch.randn(T, hidden, generator=g, device=device)).bfloat16()
+    gam = (1 + 0.3 * torch.randn(hidden, generator=g, device=device)).bfloat16()
+    gq, gk = ((1 + 0.1 * torch.randn(D, generator=g, device=device)).bfloat16() for _ in range(2))
+    cos, sin = (torch.randn(T, D, generator=g, device=device).bfloat16() for _ in range(2))
+    heads = (Hq, Hkv, Hkv)
+    if int4:
+        w = [(torch.randint(-2**31, 2**31 - 1, (hidden // 8, h * D), generator=g, device=device).int(),
+              (0.005 + 0.015 * torch.rand(hidden // 64, h * D, generator=g, device=device)).half(),
+              torch.randint(-2**31, 2**31 - 1, (hidden // 64, h * D // 8), generator=g, device=device).int())
+             for h in heads]
+        flat = [t.data_ptr() for trio in w for t in trio] + [64, _native.MQK_SCALE_FP16]
+    else:
+        w = [(0.02 * torch.randn(h * D, hidden, generator=g, device=device)).bfloat16() for h in heads]
+        flat = [t.data_ptr() for t in w]
+    ext = _native.FusedExt(in_gamma=gam.data_ptr(), in_eps=1e-6)
+    full = int(lib.mqk_fused_qkv_rope_ex_workspace_size(T, Hq, Hkv, hidden, ctypes.byref(ext)))
+    least = _native.least_workspace_bytes(T, Hq, Hkv, hidden, D, ext)
+    entry = lib.mqk_fused_qkv_rope_ex_w4a16 if int4 else lib.mqk_fused_qkv_rope_ex_bf16
+
+    def run(nbytes):
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        out = [torch.zeros(T, h, D, dtype=torch.bfloat16, device=device) for h in heads]
+        stream = int(torch.cuda.current_stream().cuda_stream)
+        st = entry(x.data_ptr(), *flat, gq.data_ptr(), gk.data_ptr(), cos.data_ptr(), sin.data_ptr(), None, T, T,
+                   hidden, Hq, Hkv, D, T, 1e-6, *(o.data_ptr() for o in out), ctypes.byref(ext), ws.data_ptr(), nbytes,
+                   stream)
+        _native.check(st, "ex")
+        torch.cuda.synchronize()
+        # the arrival counters (their statistics word aside) are zero again
+        words = ws[: _native._COUNTER_BYTES].view(torch.int32)
+        assert int(words[:1024].abs().sum()) == 0 and int(words[1024 + 64:].abs().sum()) == 0
+        return out, (x, w, gam)
+    return run, full, least
+
+
+@pytest.mark.parametrize("T,hidden,Hq,Hkv,int4", [
+    (1, 192, 2, 1, False), (3, 2112, 4, 2, False), (64, 1024, 16, 8, False), (65, 1024, 16, 8, False),
+    (129, 16384, 2, 1, False), (333, 2048, 32, 4, False), (700, 4096, 32, 8, False),
+    (1, 192, 2, 1, True), (17, 4096, 32, 8, True), (70, 1024, 16, 8, True), (257, 2048, 32, 4, True)])
+def test_both_forms_agree(T, hidden, Hq, Hkv, int4, device):
+    run, full, least = _call(T, hidden, Hq, Hkv, int4, 77 + T + hidden, device)
+    assert full > least
+    ahead, _ = run(full)
+    staged, _ = run(least)
+    for name, a, b in zip("qkv", ahead, staged):
+        a, b = a.float(), b.float()
+        assert torch.isfinite(a).all()
+        assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-3 * b.square().mean().sqrt().clamp(min=1.0)).all()), name
+
+
+def test_rows_are_the_rounded_norm(device):
+    """One-hot V rows copy normalised activations out: the 64-bit norm rounded twice
+    to bf16, except where the fp32 scale's last bits flip the first rounding (under
+    0.5 % of them): one ulp there, and the product with gamma (below 2) can make it
+    two."""
+    T, hidden, Hq, Hkv = 40, 1024, 2, 8
+    import mqk
+    g = torch.Generator(device=device).manual_seed(5)
+    x = (3 * torch.randn(1, T, hidden, generator=g, device=device)).bfloat16()
+    gam = (1 + 0.3 * torch.randn(hidden, generator=g, device=device)).bfloat16()
+    wq = torch.randn(Hq * D, hidden, generator=g, device=device).bfloat16()
+    wk = torch.randn(Hkv * D, hidden, generator=g, device=device).bfloat16()
+    wv = torch.eye(hidden, device=device).bfloat16()
+    one = torch.ones(D, dtype=torch.bfloat16, device=device)
+    cos = torch.ones(T, D, dtype=torch.bfloat16, device=device)
+    _, _, v = mqk.fused_qkv_rope_ex(x, wq, wk, wv, one, one, cos, cos, input_norm_w=gam)
+    xd = x[0].double()
+    y = (xd * torch.rsqrt(xd.square().mean(-1, keepdim=True) + 1e-6)).bfloat16()
+    want = (gam.double() * y.double()).bfloat16()
+    diff = (v.reshape(T, hidden).view(torch.int16).int() - want.view(torch.int16).int()).abs()
+    assert int(diff.max()) <= 2 and float((diff > 0).float().mean()) < 5e-3
+
+
+def test_capture_in_a_workspace_of_the_scales_only(device):
+    """Captured with a buffer that holds the plan and the per-token scales but not
+    the rows: the call is accepted and replays (it was before rows were written
+    ahead), with the eager call's values."""
+    import mqk
+    from mqk import _native
+    T, hidden, Hq, Hkv = 64, 1024, 16, 8
+    g = torch.Generator(device=device).manual_seed(6)
+    ws = [(0.02 * torch.randn(h * D, hidden, generator=g, device=device)).bfloat16() for h in (Hq, Hkv, Hkv)]
+    one = torch.ones(D, dtype=torch.bfloat16, device=device)
+    cos = torch.randn(T, D, generator=g, device=device).bfloat16()
+    gam = (1 + 0.3 * torch.randn(hidden, generator=g, device=device)).bfloat16()
+    x = torch.randn(1, T, hidden, generator=g, device=device).bfloat16()
+    call = lambda: mqk.fused_qkv_rope_ex(x, *ws, one, one, cos, cos, input_norm_w=gam)
+    want = call()
+    stream = torch.cuda.Stream(device)
+    ext = _native.FusedExt(in_gamma=gam.data_ptr(), in_eps=1e-6)
+    least = _native.least_workspace_bytes(T, Hq, Hkv, hidden, D, ext)
+    with torch.cuda.stream(stream):
+        _native._workspaces[(device.index or 0, int(stream.cuda_stream))] = torch.zeros(least, dtype=torch.uint8,
+                                                                                       device=device)
+        stream.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            out = call()
+    for _ in range(3):
+        for t in out:
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(out, want):
+            assert bool(((a.float() - b.float()).abs() <= 2.0 ** -7 * b.float().abs() + 1e-3).all())
+    _native._workspaces.pop((device.index or 0, int(stream.cuda_stream)))
