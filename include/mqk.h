@@ -129,9 +129,10 @@ int mqk_fused_qkv_rope_f32(const float* x, const float* w_q, const float* w_k, c
 /*
  * fp16 twin of mqk_fused_qkv_rope_f32 (the reference op on fp16 tensors, e.g. a
  * model loaded with dtype=float16, mini_qwen/model/loader.py:12-52): every
- * float input fp16, q / k / v written in fp16.  The fp32 front's kernel with
- * fp16 tiles on the fp16 matrix cores (exact products, fp32 sums); norm and
- * RoPE in fp32; one fp16 rounding per output.  Deliberate differences: the
+ * float input fp16, q / k / v written in fp16.  The bf16 entry point's tile kernels
+ * on the fp16 matrix cores (the fp32 front's kernel where hidden % 64 != 0 or a
+ * table is not 16-byte aligned): exact products, fp32 sums; norm and RoPE in fp32;
+ * one fp16 rounding per output.  Deliberate differences: the
  * reference rounds the fp16 GEMM output before the norm (:167-169) and Q / K to
  * bf16 before the fp16 store (:117-120); neither rounding happens here.  Same
  * validation; no workspace.
@@ -140,6 +141,17 @@ int mqk_fused_qkv_rope_f16(const mqk_f16* x, const mqk_f16* w_q, const mqk_f16* 
                            const mqk_f16* q_gamma, const mqk_f16* k_gamma, const mqk_f16* cos, const mqk_f16* sin,
                            const int32_t* positions, int64_t T, int64_t S, int64_t hidden, int Hq, int Hkv,
                            int D, int64_t cos_rows, float eps, mqk_f16* q, mqk_f16* k, mqk_f16* v, void* stream);
+
+/* mqk_fused_qkv_rope_f16 with a workspace, which lets it take the launches that
+ * exchange data through one: at least mqk_fused_qkv_rope_f16_workspace_size(T, Hq,
+ * Hkv, hidden, D) bytes (Hq, Hkv head counts), zero-filled once and not shared by
+ * overlapping calls, as for the bf16 entry point; with less it runs as without. */
+size_t mqk_fused_qkv_rope_f16_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden, int head_dim);
+int mqk_fused_qkv_rope_f16_ws(const mqk_f16* x, const mqk_f16* w_q, const mqk_f16* w_k, const mqk_f16* w_v,
+                              const mqk_f16* q_gamma, const mqk_f16* k_gamma, const mqk_f16* cos, const mqk_f16* sin,
+                              const int32_t* positions, int64_t T, int64_t S, int64_t hidden, int Hq, int Hkv,
+                              int D, int64_t cos_rows, float eps, mqk_f16* q, mqk_f16* k, mqk_f16* v,
+                              void* workspace, size_t ws_bytes, void* stream);
 
 /* Workspace bytes needed by mqk_fused_qkv_rope_bf16 / _w4a16 for these sizes
  * (0 when the chosen kernels need none; pair tiles need 66 KiB per pair of

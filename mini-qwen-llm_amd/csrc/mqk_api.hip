@@ -200,11 +200,13 @@ int plan_tile_split(int64_t M, int64_t K, int n_tiles, const Topology& topo, boo
 }
 
 Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const Topology& topo,
-                bool allow_blocks = true, bool in_norm = false, bool allow_split = true, bool allow_pair = false) {
+                bool allow_blocks = true, bool in_norm = false, bool allow_split = true, bool allow_pair = false,
+                int half = 0) {
   allow_pair = allow_pair && !int4 && aligned && g_pair_tiles.load() != 0;
   Plan pl;
   const int64_t cus = topo.cus;
-  if (use_decode(M) && aligned) {
+  if (half) allow_blocks = allow_split = false;  // (fp16 runs on the tile kernels only)
+  if (use_decode(M) && aligned && !half) {
     pl.splits = decode_splits_for(M, K, n_tiles, int(g_decode_splits.load()), topo.cus, topo.xcds);
     if (pl.splits > 0) {
       pl.tail = M;
@@ -259,7 +261,7 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
   //   launch, e.g. hidden 5120 at T = 384 / 512: 98 us against 119 / 158).
   const TileVariant* hv = nullptr;
   double head_us = 1e30;
-  if (aligned && M > 64 && g_prefill_tile.load() == 0 && g_head_tiles.load() != 0) {
+  if (aligned && (M > 64 || half) && g_prefill_tile.load() == 0 && g_head_tiles.load() != 0) {
     const int64_t t64 = (M + 63) / 64 * n_tiles, t128 = (M + 127) / 128 * n_tiles;
     const double stages = double(K / 64);
     const bool one64 = t64 <= cus, one128 = t128 <= cus;
@@ -314,8 +316,8 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
     pl.v = pv;
     return pl;
   }
-  pl.v = choose_tile_variant(int(g_prefill_tile.load()), M, n_tiles, int4, topo.cus, allow_pair);
-  if (!pl.v || !g_tail_split.load() || !aligned || M <= 64) return pl;
+  pl.v = choose_tile_variant(int(g_prefill_tile.load()), M, n_tiles, int4, topo.cus, allow_pair, half);
+  if (half || !pl.v || !g_tail_split.load() || !aligned || M <= 64) return pl;
   const int64_t r = M % pl.v->bm;
   if (r == 0 || r > 64 || !use_decode(r)) return pl;
   const int64_t rounds_all = (tile_count(*pl.v, M, n_tiles) + cus - 1) / cus;
@@ -369,7 +371,7 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     // also fits the LDS beside their ring, whichever form the workspace allows)
     const bool pair_lds = tile_dma_lds_bytes(28) + p.K * 2 <= 160 * 1024;
     const bool pairs = pair_lds && pair_tiles_ok(e);
-    const Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true, pairs);
+    const Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true, pairs, p.half);
     const size_t off = align_up(plan_region(pl, p.M, p.n_tiles), 256);
     if (ws_bytes >= off + norm_ahead_bytes(p.M, p.K)) {
       uint16_t* xn = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
@@ -384,7 +386,8 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
   p.cus = topo.cus;
   p.xcds = topo.xcds;
   const bool pair_ok = allow_pair && pair_tiles_ok(e);
-  Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, true, pair_ok);
+  Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, true, pair_ok,
+                       p.half);
   if (!pl.v && pl.splits == 0)
     return fail(MQK_ERR_BAD_OPTION, "prefill_tile variant %lld cannot run this problem (%d heads%s)",
                 (long long)g_prefill_tile.load(), p.n_tiles, int4 ? ", int4 weights" : "");
@@ -396,14 +399,14 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
   const bool split_ok = epilogue_aligned(e) && !(p.in_gamma && pl.v && tile_dma_lds_bytes(pl.v->id) + p.K * 2 > 160 * 1024);
   if (pl.ksplit > 0 && (!fits(base) || !split_ok)) {
     // a workspace sized without the split-K tile launch (or operands it cannot take): plan without it
-    pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, false, pair_ok);
+    pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, false, pair_ok, p.half);
     base = region(pl);
   }
   if (pl.v && is_pair_variant(pl.v->id) &&
       (!fits(base) || (p.in_gamma && tile_dma_lds_bytes(pl.v->id) + p.K * 2 > 160 * 1024))) {
     // a workspace sized without the pair tiles' exchange area, or an input norm whose
     // gamma does not fit the LDS beside their ring: plan without them
-    pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, false, false);
+    pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, false, false, p.half);
     base = region(pl);
   }
   while (!pl.v && pl.passes > 1 && !fits(base)) {
@@ -855,7 +858,8 @@ int mqk_fused_qkv_rope_bf16(const mqk_bf16* x, const mqk_bf16* w_q, const mqk_bf
 static int fused_f32_impl(bool half, const void* x, const void* w_q, const void* w_k, const void* w_v,
                           const void* q_gamma, const void* k_gamma, const void* cos, const void* sin,
                           const int32_t* positions, int64_t T, int64_t S, int64_t hidden, int Hq, int Hkv, int D,
-                          int64_t cos_rows, float eps, void* q, void* k, void* v, void* stream) {
+                          int64_t cos_rows, float eps, void* q, void* k, void* v, void* workspace, size_t ws_bytes,
+                          void* stream) {
   if (T < 0 || hidden <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0)
     return fail(MQK_ERR_BAD_SHAPE, "need T >= 0, hidden > 0, Hq > 0, Hkv > 0, D > 0");
   if (int st = check_head_dim(D, Hq, Hkv); st != MQK_OK) return st;
@@ -872,6 +876,26 @@ static int fused_f32_impl(bool half, const void* x, const void* w_q, const void*
   int st = check_rope_args(q_gamma, k_gamma, cos, sin, S, cos_rows, positions, eps);
   if (st != MQK_OK) return st;
   to_blocks(D, Hq, Hkv);
+  if (half && hidden % kBK == 0 && aligned16(q_gamma) && aligned16(k_gamma) && aligned16(cos) && aligned16(sin)) {
+    // fp16 with whole 64-k stages and 16-byte table rows: the pipelined tile kernels
+    // (one call at hidden 4096, 32 / 8 heads on MI355X: T = 1 50.7 us in the kernel
+    // below, 29.8 here; T = 2048 306 and 102).  Other hidden sizes (multiples of 32) and
+    // unaligned tables stay below.
+    auto u = [](const void* ptr) { return static_cast<const uint16_t*>(ptr); };
+    auto o = [](void* ptr) { return static_cast<uint16_t*>(ptr); };
+    ProblemArgs p{u(x), T, hidden, Hq + 2 * Hkv};
+    p.half = 1;
+    WeightArgs w{};
+    w.w[0] = u(w_q);
+    w.w[1] = u(w_k);
+    w.w[2] = u(w_v);
+    w.n_cols[0] = int64_t(Hq) * kHeadDim;
+    w.n_cols[1] = w.n_cols[2] = int64_t(Hkv) * kHeadDim;
+    EpilogueArgs e = make_qkv_epilogue(u(q_gamma), u(k_gamma), u(cos), u(sin), positions, S, cos_rows, eps, o(q), o(k),
+                                       o(v), Hq, Hkv);
+    e.head_dim = D;
+    return run_fused(0, p, w, e, 0.f, workspace, ws_bytes, static_cast<hipStream_t>(stream));
+  }
   F32Args a{};
   a.head_dim = D;
   a.x = x;
@@ -905,7 +929,26 @@ int mqk_fused_qkv_rope_f32(const float* x, const float* w_q, const float* w_k, c
                            const int32_t* positions, int64_t T, int64_t S, int64_t hidden, int Hq, int Hkv,
                            int D, int64_t cos_rows, float eps, float* q, float* k, float* v, void* stream) {
   return fused_f32_impl(false, x, w_q, w_k, w_v, q_gamma, k_gamma, cos, sin, positions, T, S, hidden, Hq, Hkv, D,
-                        cos_rows, eps, q, k, v, stream);
+                        cos_rows, eps, q, k, v, nullptr, 0, stream);
+}
+
+size_t mqk_fused_qkv_rope_f16_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden, int head_dim) {
+  if (T <= 0 || Hq <= 0 || Hkv <= 0 || hidden <= 0 || hidden % kBK != 0 || (head_dim != kHeadDim && head_dim != 64))
+    return 0;
+  to_blocks(head_dim, Hq, Hkv);
+  const int tiles = Hq + 2 * Hkv;
+  if (tiles < 1 || tiles > kMaxTiles) return 0;
+  const Plan pl = plan_fused(0, T, hidden, tiles, true, device_topology(), true, false, true, head_dim == kHeadDim, 1);
+  return pl.splits > 0 || (pl.v && is_pair_variant(pl.v->id)) ? plan_region(pl, T, tiles) : 0;
+}
+
+int mqk_fused_qkv_rope_f16_ws(const mqk_f16* x, const mqk_f16* w_q, const mqk_f16* w_k, const mqk_f16* w_v,
+                              const mqk_f16* q_gamma, const mqk_f16* k_gamma, const mqk_f16* cos, const mqk_f16* sin,
+                              const int32_t* positions, int64_t T, int64_t S, int64_t hidden, int Hq, int Hkv, int D,
+                              int64_t cos_rows, float eps, mqk_f16* q, mqk_f16* k, mqk_f16* v, void* workspace,
+                              size_t ws_bytes, void* stream) {
+  return fused_f32_impl(true, x, w_q, w_k, w_v, q_gamma, k_gamma, cos, sin, positions, T, S, hidden, Hq, Hkv, D,
+                        cos_rows, eps, q, k, v, workspace, ws_bytes, stream);
 }
 
 int mqk_fused_qkv_rope_f16(const mqk_f16* x, const mqk_f16* w_q, const mqk_f16* w_k, const mqk_f16* w_v,
@@ -913,7 +956,7 @@ int mqk_fused_qkv_rope_f16(const mqk_f16* x, const mqk_f16* w_q, const mqk_f16* 
                            const int32_t* positions, int64_t T, int64_t S, int64_t hidden, int Hq, int Hkv,
                            int D, int64_t cos_rows, float eps, mqk_f16* q, mqk_f16* k, mqk_f16* v, void* stream) {
   return fused_f32_impl(true, x, w_q, w_k, w_v, q_gamma, k_gamma, cos, sin, positions, T, S, hidden, Hq, Hkv, D,
-                        cos_rows, eps, q, k, v, stream);
+                        cos_rows, eps, q, k, v, nullptr, 0, stream);
 }
 
 // ---- allocation-free variant of mqk_fused_qkv_rope_bf16 ---------------------------------

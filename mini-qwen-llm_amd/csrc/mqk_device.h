@@ -64,6 +64,26 @@ __device__ __forceinline__ f32x4_t mfma_16x16x32(u32x4_t a, u32x4_t b, f32x4_t c
                                                  __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
 }
 
+// The two 16-bit element types of the tile and decode kernels: conversions and the
+// 16 x 16 x 32 MFMA of that type (exact products, fp32 sums; the same lane layout).
+struct Bf16 {
+  static __device__ __forceinline__ float to_f32(uint32_t bits16) { return bf16_to_f32(bits16); }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) { return pack_bf16x2(a, b); }
+  static __device__ __forceinline__ f32x4_t mfma(u32x4_t a, u32x4_t b, f32x4_t c) { return mfma_16x16x32(a, b, c); }
+};
+struct Fp16 {
+  static __device__ __forceinline__ float to_f32(uint32_t bits16) { return f16_to_f32(bits16); }
+  static __device__ __forceinline__ uint32_t pack2(float a, float b) {  // round to nearest even
+    typedef _Float16 f16x2_v __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, (f16x2_v){static_cast<_Float16>(a), static_cast<_Float16>(b)});
+  }
+  static __device__ __forceinline__ f32x4_t mfma(u32x4_t a, u32x4_t b, f32x4_t c) {
+    typedef _Float16 f16x8_v __attribute__((ext_vector_type(8)));
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8_v, a), __builtin_bit_cast(f16x8_v, b), c, 0,
+                                                  0, 0);
+  }
+};
+
 // Dequantize one packed int32 (8 consecutive k of one output column) to 8 bf16:
 // w = (q - z) * s, exact in fp32 (|q - z| <= 15 times an 8/11-bit mantissa),
 // then one rounding to bf16.  Nibble e holds k = 8j + e (little-endian nibbles).

@@ -68,7 +68,7 @@ struct EpilogueArgs {
 };
 
 struct ProblemArgs {
-  const uint16_t* x;   // [M, K] bf16
+  const uint16_t* x;   // [M, K] bf16 (or fp16, see half)
   int64_t M;
   int64_t K;
   int n_tiles;         // number of 128-column tiles (heads)
@@ -81,6 +81,9 @@ struct ProblemArgs {
   // b % xcds.
   int cus;
   int xcds;
+  // Element type of x, the weights, gamma / cos / sin and the outputs: 0 bf16, 1 fp16
+  // (the tile variants fp16_variant() names; no input norm).
+  int half = 0;
 };
 
 // One tile-kernel variant: BM rows x (HPT*128) columns per workgroup, with KZ
@@ -98,8 +101,12 @@ const TileVariant* tile_variant(int index);
 // Picks a variant for the problem (id 0 = automatic).
 // allow_pair: the pair-tile variants (24-28) may be chosen (bf16 q/k/v outputs
 // with head_dim 128 and a workspace for their exchange).
+// half: fp16 elements (a requested variant without an fp16 form counts as automatic).
 const TileVariant* choose_tile_variant(int requested_id, int64_t M, int n_tiles, int int4, int cus,
-                                       bool allow_pair = false);
+                                       bool allow_pair = false, int half = 0);
+inline bool fp16_variant(int id) {
+  return id == 16 || id == 18 || id == 20 || id == 21 || id == 23 || id == 25 || id == 26 || id == 28;
+}
 // Workgroups of one launch of variant v over M rows and n_tiles heads.
 int64_t tile_count(const TileVariant& v, int64_t M, int n_tiles);
 hipError_t launch_tile(const TileVariant& v, int int4, const ProblemArgs& p, const WeightArgs& w,

@@ -460,7 +460,9 @@ int64_t tile_count(const TileVariant& v, int64_t M, int n_tiles) {
   return ((M + v.bm - 1) / v.bm) * (n_tiles / v.hpt) * (is_pair_variant(v.id) ? 2 : 1);
 }
 
-const TileVariant* choose_tile_variant(int requested_id, int64_t M, int n_tiles, int int4, int cus_, bool allow_pair) {
+const TileVariant* choose_tile_variant(int requested_id, int64_t M, int n_tiles, int int4, int cus_, bool allow_pair,
+                                       int half) {
+  if (half && !fp16_variant(requested_id)) requested_id = 0;
   // (a pair launch has one exchange word per pair in the workspace's kSplitMaxTiles lines)
   auto pair_fits = [&](const TileVariant& v) { return allow_pair && tile_count(v, M, n_tiles) / 2 <= kSplitMaxTiles; };
   if (requested_id > 0) {
@@ -498,8 +500,14 @@ const TileVariant* choose_tile_variant(int requested_id, int64_t M, int n_tiles,
   // (33 is 31 with waves of 256 x 32, so every int4 weight is dequantised once per
   // workgroup instead of twice: 419 us against 447 us on the W4A16 ragged batch)
   static const Cand int4_cands[] = {{33, 1.07f}, {31, 1.00f}, {30, 0.75f}, {32, 0.54f}};
-  const Cand* cands = int4 ? int4_cands : bf16_cands;
-  const int ncand = int(int4 ? sizeof(int4_cands) / sizeof(int4_cands[0]) : sizeof(bf16_cands) / sizeof(bf16_cands[0]));
+  // (fp16: the bf16 shapes that have an fp16 form, at the bf16 rates; 21, 128 x 128 with
+  // 8 waves, is the one that tiles any head count)
+  static const Cand f16_cands[] = {{16, 1.00f}, {18, 1.27f}, {23, 0.90f}, {25, 1.33f},
+                                   {26, 0.82f}, {28, 0.91f}, {21, 0.65f}};
+  const Cand* cands = int4 ? int4_cands : (half ? f16_cands : bf16_cands);
+  const int ncand = int(int4 ? sizeof(int4_cands) / sizeof(int4_cands[0])
+                             : (half ? sizeof(f16_cands) / sizeof(f16_cands[0])
+                                     : sizeof(bf16_cands) / sizeof(bf16_cands[0])));
   const int64_t cus = cus_ > 0 ? cus_ : 256;
   const TileVariant* best = find_variant(1);
   float best_score = -1.f;

@@ -42,15 +42,16 @@ constexpr int kEpiPitch = kHeadDim + 4;     // fp32 pitch of the epilogue head t
 // RMSNorm (fused_qkv_rope.py:98-100) then rotate-half RoPE (:102-118) of the
 // dim pair (d, d+64); gl / gh are the gammas of d / d+64 and element
 // (wd, sh) of the cos / sin registers holds the table values of d and d+64.
+template <class E = Bf16>
 __device__ __forceinline__ void norm_rope_pair(float& lo, float& hi, float rms, float gl, float gh,
                                                const u32x4_t (&c2)[2], const u32x4_t (&s2)[2], int wd, int sh) {
 #pragma clang fp contract(off)
   const float x1n = lo * rms * gl;
   const float x2n = hi * rms * gh;
-  const float co1 = bf16_to_f32((c2[0][wd] >> sh) & 0xFFFFu);
-  const float co2 = bf16_to_f32((c2[1][wd] >> sh) & 0xFFFFu);
-  const float si1 = bf16_to_f32((s2[0][wd] >> sh) & 0xFFFFu);
-  const float si2 = bf16_to_f32((s2[1][wd] >> sh) & 0xFFFFu);
+  const float co1 = E::to_f32((c2[0][wd] >> sh) & 0xFFFFu);
+  const float co2 = E::to_f32((c2[1][wd] >> sh) & 0xFFFFu);
+  const float si1 = E::to_f32((s2[0][wd] >> sh) & 0xFFFFu);
+  const float si2 = E::to_f32((s2[1][wd] >> sh) & 0xFFFFu);
   lo = __builtin_fmaf(x1n, co1, -(x2n * si1));
   hi = __builtin_fmaf(x2n, co2, x1n * si2);
 }
@@ -157,7 +158,7 @@ template <> struct AccBlock<f32x4_t> {
 // cslot[q] its paged-KV-cache slot (-1: none).
 // units: bit u set = rows [32u, 32u+32) of the tile are stored (the split-K
 // launch finishes a tile's rows in 32-row units spread over its workgroups).
-template <int BM, int NH, int WM, int WN, int THREADS, int MB, int NB, class AV, class RowV, class SlotV>
+template <class E, int BM, int NH, int WM, int WN, int THREADS, int MB, int NB, class AV, class RowV, class SlotV>
 __device__ __forceinline__ void tile_epilogue(const AV (&acc)[MB][NB], const RowV& prow,
                                               const SlotV& cslot, int head0, int64_t m0, const ProblemArgs& p,
                                               const EpilogueArgs& e, unsigned char* smem,
@@ -236,8 +237,8 @@ __device__ __forceinline__ void tile_epilogue(const AV (&acc)[MB][NB], const Row
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int wd = i >> 1, sh = (i & 1) * 16;
-        g1[i] = bf16_to_f32((g[0][wd] >> sh) & 0xFFFFu);
-        g2[i] = bf16_to_f32((g[1][wd] >> sh) & 0xFFFFu);
+        g1[i] = E::to_f32((g[0][wd] >> sh) & 0xFFFFu);
+        g2[i] = E::to_f32((g[1][wd] >> sh) & 0xFFFFu);
       }
     }
 #pragma unroll
@@ -275,17 +276,17 @@ __device__ __forceinline__ void tile_epilogue(const AV (&acc)[MB][NB], const Row
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int wd = i >> 1, sh = (i & 1) * 16;
-          const float gl = kHoistGamma ? g1[i] : bf16_to_f32((g[0][wd] >> sh) & 0xFFFFu);
-          const float gh = kHoistGamma ? g2[i] : bf16_to_f32((g[1][wd] >> sh) & 0xFFFFu);
-          norm_rope_pair(lo[i], hi[i], rms, gl, gh, c2, s2, wd, sh);
+          const float gl = kHoistGamma ? g1[i] : E::to_f32((g[0][wd] >> sh) & 0xFFFFu);
+          const float gh = kHoistGamma ? g2[i] : E::to_f32((g[1][wd] >> sh) & 0xFFFFu);
+          norm_rope_pair<E>(lo[i], hi[i], rms, gl, gh, c2, s2, wd, sh);
         }
       }
       if (t < p.M && ((units >> (r0 >> 5)) & 1u)) {
         u32x4_t o1, o2;
-        o1.x = pack_bf16x2(lo[0], lo[1]); o1.y = pack_bf16x2(lo[2], lo[3]);
-        o1.z = pack_bf16x2(lo[4], lo[5]); o1.w = pack_bf16x2(lo[6], lo[7]);
-        o2.x = pack_bf16x2(hi[0], hi[1]); o2.y = pack_bf16x2(hi[2], hi[3]);
-        o2.z = pack_bf16x2(hi[4], hi[5]); o2.w = pack_bf16x2(hi[6], hi[7]);
+        o1.x = E::pack2(lo[0], lo[1]); o1.y = E::pack2(lo[2], lo[3]);
+        o1.z = E::pack2(lo[4], lo[5]); o1.w = E::pack2(lo[6], lo[7]);
+        o2.x = E::pack2(hi[0], hi[1]); o2.y = E::pack2(hi[2], hi[3]);
+        o2.z = E::pack2(hi[4], hi[5]); o2.w = E::pack2(hi[6], hi[7]);
         if (e.qkv) {
           const int H = proj == 0 ? e.Hq : e.Hkv;
           uint16_t* base = proj == 0 ? e.q : (proj == 1 ? e.k : e.v);  // k / v may be null (cache only)
@@ -432,7 +433,7 @@ struct PairX {
 // then bit 2 + side); the partner, arriving later, sees that bit and finishes both
 // halves.  Published data uses agent-scope (device-coherent) stores and loads, so
 // the two sides may run on any XCDs.  V heads (and plain outputs) need no exchange.
-template <int BM, int NH, int WM, int WN, int THREADS, int MB, int NB, class AV, class RowV, class SlotV>
+template <class E, int BM, int NH, int WM, int WN, int THREADS, int MB, int NB, class AV, class RowV, class SlotV>
 __device__ __forceinline__ void pair_epilogue(const AV (&acc)[MB][NB], RowV prow, SlotV cslot,
                                               int h_pair, int side, int pair, int64_t m0, const ProblemArgs& p,
                                               const EpilogueArgs& e, unsigned char* smem, const PairX& px) {
@@ -525,16 +526,16 @@ __device__ __forceinline__ void pair_epilogue(const AV (&acc)[MB][NB], RowV prow
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           const int wd = i >> 1, sh = (i & 1) * 16;
-          norm_rope_pair(lo[i], hi[i], rms, bf16_to_f32((g0[wd] >> sh) & 0xFFFFu),
-                         bf16_to_f32((g1[wd] >> sh) & 0xFFFFu), c2, s2, wd, sh);
+          norm_rope_pair<E>(lo[i], hi[i], rms, E::to_f32((g0[wd] >> sh) & 0xFFFFu),
+                         E::to_f32((g1[wd] >> sh) & 0xFFFFu), c2, s2, wd, sh);
         }
       }
       if (!valid) continue;
       u32x4_t o1, o2;
-      o1.x = pack_bf16x2(lo[0], lo[1]); o1.y = pack_bf16x2(lo[2], lo[3]);
-      o1.z = pack_bf16x2(lo[4], lo[5]); o1.w = pack_bf16x2(lo[6], lo[7]);
-      o2.x = pack_bf16x2(hi[0], hi[1]); o2.y = pack_bf16x2(hi[2], hi[3]);
-      o2.z = pack_bf16x2(hi[4], hi[5]); o2.w = pack_bf16x2(hi[6], hi[7]);
+      o1.x = E::pack2(lo[0], lo[1]); o1.y = E::pack2(lo[2], lo[3]);
+      o1.z = E::pack2(lo[4], lo[5]); o1.w = E::pack2(lo[6], lo[7]);
+      o2.x = E::pack2(hi[0], hi[1]); o2.y = E::pack2(hi[2], hi[3]);
+      o2.z = E::pack2(hi[4], hi[5]); o2.w = E::pack2(hi[6], hi[7]);
       const int H = proj == 0 ? e.Hq : e.Hkv;
       uint16_t* obase = pick3<uint16_t>(proj, e.q, e.k, e.v);  // k / v may be null (cache only)
       if (obase) {
@@ -552,7 +553,7 @@ __device__ __forceinline__ void pair_epilogue(const AV (&acc)[MB][NB], RowV prow
   };
 
   if (!qk) {  // a V head: each side stores its half as it is
-    tile_epilogue<BM, NH, WM, WN, THREADS>(acc, prow, cslot, head0, m0, p, e, smem);
+    tile_epilogue<E, BM, NH, WM, WN, THREADS>(acc, prow, cslot, head0, m0, p, e, smem);
     stage_half();
     __syncthreads();
     finish_half(side, nullptr);
@@ -581,7 +582,7 @@ __device__ __forceinline__ void pair_epilogue(const AV (&acc)[MB][NB], RowV prow
   __syncthreads();
   const uint32_t seen = xword;
   // ---- the whole heads (their barriers separate the reads of xword from its next write)
-  tile_epilogue<BM, NH, WM, WN, THREADS>(acc, prow, cslot, head0, m0, p, e, smem);
+  tile_epilogue<E, BM, NH, WM, WN, THREADS>(acc, prow, cslot, head0, m0, p, e, smem);
   bool other_half = false, clear = false;
   if (seen & p_other) {
     // the partner published first: it clears the word, unless it handed its half over
@@ -651,9 +652,10 @@ __device__ __forceinline__ void pair_epilogue(const AV (&acc)[MB][NB], RowV prow
 // [h0, h0 + 2*NH + 1) of a pair are covered by two workgroups, side 0 holding
 // heads h0 .. h0+NH-1 and half of head h0+NH, side 1 the other half of that head
 // and heads h0+NH+1 .. h0+2NH; pair_epilogue finishes the shared head.
-template <int BM, int NH, int WM, int WN, int NS, int SBK, int XC = 0>
-__global__ void __launch_bounds__(WM* WN * 64)
-tile_dma_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, int group_m, PairX px) {
+// E: the element type of x, the weights, gamma / cos / sin and the outputs.
+template <class E, int BM, int NH, int WM, int WN, int NS, int SBK, int XC>
+__device__ __forceinline__ void tile_dma_body(const ProblemArgs& p, const WeightArgs& w, const EpilogueArgs& e,
+                                              int group_m, const PairX& px) {
   using S = DmaShape<BM, NH, WM, WN, NS, SBK, XC>;
   constexpr int kRowBytes = S::kRowBytes;
   __shared__ __attribute__((aligned(16))) unsigned char smem[S::kLdsBytes];
@@ -748,7 +750,7 @@ tile_dma_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, int group_m, PairX 
   }
   // input RMSNorm: scale of the x row and k offset of the chunk each of this
   // lane's x loads brings in (load i < kALoads, row0 + lane / chunks, slot lane % chunks)
-  const bool in_norm = p.in_gamma != nullptr;
+  const bool in_norm = std::is_same<E, Bf16>::value && p.in_gamma != nullptr;
   float a_scale[S::kALoads];
   int a_koff[S::kALoads];
 #pragma unroll
@@ -819,15 +821,31 @@ tile_dma_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, int group_m, PairX 
 #pragma unroll
       for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < kNB; ++nb) acc[mb][nb] = mfma_16x16x32(af[mb], bf[nb], acc[mb][nb]);
+        for (int nb = 0; nb < kNB; ++nb) acc[mb][nb] = E::mfma(af[mb], bf[nb], acc[mb][nb]);
     }
   }
   barrier();  // every wave is done with the ring; the epilogue reuses the LDS
 
   if constexpr (XC != 0)
-    pair_epilogue<BM, NH, WM, WN, S::kThreads>(acc, prow, cslot, h_pair, side, mt * n_ht + ht, m0, p, e, smem, px);
+    pair_epilogue<E, BM, NH, WM, WN, S::kThreads>(acc, prow, cslot, h_pair, side, mt * n_ht + ht, m0, p, e, smem, px);
   else
-    tile_epilogue<BM, NH, WM, WN, S::kThreads>(acc, prow, cslot, head0, m0, p, e, smem);
+    tile_epilogue<E, BM, NH, WM, WN, S::kThreads>(acc, prow, cslot, head0, m0, p, e, smem);
+}
+
+template <int BM, int NH, int WM, int WN, int NS, int SBK, int XC = 0>
+__global__ void __launch_bounds__(WM* WN * 64)
+tile_dma_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, int group_m, PairX px) {
+  tile_dma_body<Bf16, BM, NH, WM, WN, NS, SBK, XC>(p, w, e, group_m, px);
+}
+
+// The same on fp16 tensors (ids 16, 18, 20, 21, 23, 25, 26, 28).  Bound as the bf16
+// kernel is; against the 32 x 128 register-staged tiles that ran fp16 before, one
+// call on MI355X: hidden 1024, 16 / 8 heads T = 2048 60 -> 25 us, hidden 4096, 32 / 8
+// heads T = 777 128 -> 55 us, T = 2048 306 -> 102 us.
+template <int BM, int NH, int WM, int WN, int NS, int SBK, int XC = 0>
+__global__ void __launch_bounds__(WM* WN * 64)
+tile_dma_f16_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, int group_m, PairX px) {
+  tile_dma_body<Fp16, BM, NH, WM, WN, NS, SBK, XC>(p, w, e, group_m, px);
 }
 
 // The split-K launch of the pipelined kernel (a separate kernel, so that the
@@ -1201,7 +1219,8 @@ tile_dma_split_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, TileSplit sp)
   }
 }
 
-template <int BM, int NH, int WM, int WN, int NS, int SBK = 32>
+// F16: the variant also exists for fp16 elements (p.half).
+template <int BM, int NH, int WM, int WN, int NS, int SBK = 32, bool F16 = false>
 hipError_t launch_dma(const ProblemArgs& p, const WeightArgs& w, const EpilogueArgs& e, int group_m,
                       hipStream_t stream) {
   using S = DmaShape<BM, NH, WM, WN, NS, SBK>;
@@ -1209,6 +1228,13 @@ hipError_t launch_dma(const ProblemArgs& p, const WeightArgs& w, const EpilogueA
   const int blocks = n_mt * (p.n_tiles / NH);
   const size_t dyn = p.in_gamma ? size_t(p.K) * 2 : 0;
   if (S::kLdsBytes + dyn > 160 * 1024) return hipErrorInvalidValue;
+  if (p.half) {
+    if constexpr (!F16) return hipErrorInvalidValue;
+    else
+      hipLaunchKernelGGL((tile_dma_f16_kernel<BM, NH, WM, WN, NS, SBK>), dim3(blocks), dim3(S::kThreads), 0, stream, p,
+                         w, e, group_m < 1 ? 1 : group_m, PairX{});
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((tile_dma_kernel<BM, NH, WM, WN, NS, SBK>), dim3(blocks), dim3(S::kThreads), dyn, stream, p, w, e,
                      group_m < 1 ? 1 : group_m, PairX{});
   return hipGetLastError();
@@ -1497,7 +1523,7 @@ tile_dma_w4_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, int group_m) {
     }
   }
   barrier();  // every wave is done with the ring; the epilogue reuses the LDS
-  tile_epilogue<BM, NH, WM, WN, S::kThreads>(acc, prow, cslot, ht * NH, m0, p, e, smem);
+  tile_epilogue<Bf16, BM, NH, WM, WN, S::kThreads>(acc, prow, cslot, ht * NH, m0, p, e, smem);
 }
 
 template <int BM, int NH, int WM, int WN, int NS, int SBK>
@@ -1506,7 +1532,7 @@ size_t pair_bytes(int64_t M, int n_tiles) {
   return kDecodeCounterBytes + size_t(pairs) * (2 * BM + BM * 64) * sizeof(float);
 }
 
-template <int BM, int NH, int WM, int WN, int NS, int SBK>
+template <int BM, int NH, int WM, int WN, int NS, int SBK, bool F16 = false>
 hipError_t launch_pair(const ProblemArgs& p, const WeightArgs& w, const EpilogueArgs& e, int group_m,
                        void* workspace, int max_spins, hipStream_t stream) {
   using S = DmaShape<BM, NH, WM, WN, NS, SBK, 64>;
@@ -1523,6 +1549,13 @@ hipError_t launch_pair(const ProblemArgs& p, const WeightArgs& w, const Epilogue
   px.max_spins = max_spins < 0 ? 0 : max_spins;
   px.hold = g_pair_hold & 0xFFFF;
   px.cross = g_pair_hold >> 16;
+  if (p.half) {
+    if constexpr (!F16) return hipErrorInvalidValue;
+    else
+      hipLaunchKernelGGL((tile_dma_f16_kernel<BM, NH, WM, WN, NS, SBK, 64>), dim3(unsigned(pairs * 2)),
+                         dim3(S::kThreads), 0, stream, p, w, e, group_m < 1 ? 1 : group_m, px);
+    return hipGetLastError();
+  }
   hipLaunchKernelGGL((tile_dma_kernel<BM, NH, WM, WN, NS, SBK, 64>), dim3(unsigned(pairs * 2)), dim3(S::kThreads), dyn,
                      stream, p, w, e, group_m < 1 ? 1 : group_m, px);
   return hipGetLastError();
@@ -1552,14 +1585,14 @@ hipError_t launch_tile_dma(int id, const ProblemArgs& p, const WeightArgs& w, co
     case 13: return launch_dma<128, 2, 2, 2, 4>(p, w, e, group_m, stream);   // 128x256, 4 waves
     case 14: return launch_dma<256, 2, 2, 4, 4>(p, w, e, group_m, stream);   // 256x256, 8 waves (128x64)
     case 15: return launch_dma<128, 3, 2, 4, 5>(p, w, e, group_m, stream);   // 128x384, 5 stages
-    case 16: return launch_dma<128, 3, 2, 4, 2, 64>(p, w, e, group_m, stream);  // 128x384, 2 stages of 64 k
+    case 16: return launch_dma<128, 3, 2, 4, 2, 64, true>(p, w, e, group_m, stream);  // 128x384, 2 stages of 64 k
     case 17: return launch_dma<256, 2, 4, 2, 2, 64>(p, w, e, group_m, stream);  // 256x256, 2 stages of 64 k
-    case 18: return launch_dma<256, 2, 2, 4, 2, 64>(p, w, e, group_m, stream);  // 256x256 (128x64 waves), 64 k
+    case 18: return launch_dma<256, 2, 2, 4, 2, 64, true>(p, w, e, group_m, stream);  // 256x256 (128x64 waves), 64 k
     case 19: return launch_dma<128, 1, 2, 2, 4, 64>(p, w, e, group_m, stream);  // 128x128, 4 waves, 4 stages of 64 k
-    case 20: return launch_dma<64, 1, 1, 4, 4, 64>(p, w, e, group_m, stream);   // 64x128, 4 waves (64x32)
-    case 21: return launch_dma<128, 1, 2, 4, 4, 64>(p, w, e, group_m, stream);  // 128x128, 8 waves (64x32)
+    case 20: return launch_dma<64, 1, 1, 4, 4, 64, true>(p, w, e, group_m, stream);   // 64x128, 4 waves (64x32)
+    case 21: return launch_dma<128, 1, 2, 4, 4, 64, true>(p, w, e, group_m, stream);  // 128x128, 8 waves (64x32)
     case 22: return launch_dma<256, 1, 4, 2, 3, 64>(p, w, e, group_m, stream);  // 256x128, 8 waves (64x64), 3 stages
-    case 23: return launch_dma<128, 2, 2, 4, 3, 64>(p, w, e, group_m, stream);  // 128x256, 8 waves (64x64), 3 stages
+    case 23: return launch_dma<128, 2, 2, 4, 3, 64, true>(p, w, e, group_m, stream);  // 128x256, 8 waves (64x64), 3 stages
     default: return hipErrorInvalidValue;
   }
 }
@@ -1570,10 +1603,10 @@ hipError_t launch_pair_tile(int id, const ProblemArgs& p, const WeightArgs& w, c
                             void* workspace, int max_spins, hipStream_t stream) {
   switch (id) {
     case 24: return launch_pair<256, 1, 4, 2, 2, 64>(p, w, e, group_m, workspace, max_spins, stream);  // 256x192
-    case 25: return launch_pair<256, 2, 4, 2, 2, 64>(p, w, e, group_m, workspace, max_spins, stream);  // 256x320
-    case 26: return launch_pair<128, 1, 4, 2, 3, 64>(p, w, e, group_m, workspace, max_spins, stream);  // 128x192
+    case 25: return launch_pair<256, 2, 4, 2, 2, 64, true>(p, w, e, group_m, workspace, max_spins, stream);  // 256x320
+    case 26: return launch_pair<128, 1, 4, 2, 3, 64, true>(p, w, e, group_m, workspace, max_spins, stream);  // 128x192
     case 27: return launch_pair<128, 2, 4, 2, 2, 64>(p, w, e, group_m, workspace, max_spins, stream);  // 128x320
-    case 28: return launch_pair<192, 1, 3, 2, 3, 64>(p, w, e, group_m, workspace, max_spins, stream);  // 192x192
+    case 28: return launch_pair<192, 1, 3, 2, 3, 64, true>(p, w, e, group_m, workspace, max_spins, stream);  // 192x192
     default: return hipErrorInvalidValue;
   }
 }

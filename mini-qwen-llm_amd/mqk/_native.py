@@ -82,6 +82,13 @@ SIGNATURES = {
          _I64, _I64, _I64, _I, _I, _I,           # T S hidden Hq Hkv D
          _I64, _F, _P, _P, _P, _P],              # cos_rows eps q k v stream
     ),
+    "mqk_fused_qkv_rope_f16_ws": (
+        _I,
+        [_P, _P, _P, _P, _P, _P, _P, _P, _P,     # x w_q w_k w_v q_gamma k_gamma cos sin positions
+         _I64, _I64, _I64, _I, _I, _I,           # T S hidden Hq Hkv D
+         _I64, _F, _P, _P, _P, _P, _SZ, _P],     # cos_rows eps q k v workspace ws_bytes stream
+    ),
+    "mqk_fused_qkv_rope_f16_workspace_size": (_SZ, [_I64, _I, _I, _I64, _I]),
     "mqk_fused_qkv_rope_workspace_size": (_SZ, [_I64, _I, _I, _I64]),
     "mqk_fused_qkv_rope_workspace_size_hd": (_SZ, [_I64, _I, _I, _I64, _I]),
     "mqk_fused_qkv_rope_bf16_noalloc": (
@@ -280,7 +287,7 @@ def workspace(device: torch.device, stream, nbytes: int, least=None):
         buf = _workspaces.get(key)
         if buf is None or buf.numel() < nbytes:
             if torch.cuda.is_current_stream_capturing():
-                if buf is not None and least is not None and buf.numel() >= least():
+                if least is not None and (0 if buf is None else buf.numel()) >= least():
                     return buf
                 raise MqkNativeError(
                     f"the mqk workspace of this stream must grow to {nbytes} bytes during HIP-graph "

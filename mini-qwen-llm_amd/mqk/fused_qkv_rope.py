@@ -96,6 +96,10 @@ def _rope_tables(cos, sin, D, device, dtype=torch.bfloat16):
     return cos, sin
 
 
+def _no_bytes() -> int:
+    return 0
+
+
 def fused_qkv_rope(
     x: torch.Tensor,
     w_q: torch.Tensor,
@@ -139,26 +143,31 @@ def fused_qkv_rope(
 
     lib = _native.library()
     stream = _native.stream_handle(device)
-    if dtype != torch.bfloat16:
-        entry = "mqk_fused_qkv_rope_f32" if dtype == torch.float32 else "mqk_fused_qkv_rope_f16"
+    if dtype == torch.float32:
         status = _native.call(
-            device, getattr(lib, entry),
+            device, lib.mqk_fused_qkv_rope_f32,
             x.data_ptr(), w_q.data_ptr(), w_k.data_ptr(), w_v.data_ptr(),
             q_norm_w.data_ptr(), k_norm_w.data_ptr(), cos.data_ptr(), sin.data_ptr(), _native.ptr(pos),
             T, S, H, H_Q, H_KV, D, cos.shape[0], EPS,
             q.data_ptr(), k.data_ptr(), v.data_ptr(), stream)
-        _native.check(status, entry)
+        _native.check(status, "mqk_fused_qkv_rope_f32")
         return q, k, v
-    nbytes = _native.fused_workspace_bytes(T, H_Q, H_KV, H, D)
-    ws = _native.workspace(device, stream, nbytes)
+    if dtype == torch.float16:
+        # (no workspace is needed to run: one that cannot grow during capture is passed as it is)
+        entry, least = "mqk_fused_qkv_rope_f16_ws", _no_bytes
+        nbytes = int(lib.mqk_fused_qkv_rope_f16_workspace_size(T, H_Q, H_KV, H, D))
+    else:
+        entry, least = "mqk_fused_qkv_rope_bf16", None
+        nbytes = _native.fused_workspace_bytes(T, H_Q, H_KV, H, D)
+    ws = _native.workspace(device, stream, nbytes, least)
     status = _native.call(
-        device, lib.mqk_fused_qkv_rope_bf16,
+        device, getattr(lib, entry),
         x.data_ptr(), w_q.data_ptr(), w_k.data_ptr(), w_v.data_ptr(),
         q_norm_w.data_ptr(), k_norm_w.data_ptr(), cos.data_ptr(), sin.data_ptr(), _native.ptr(pos),
         T, S, H, H_Q, H_KV, D, cos.shape[0], EPS,
         q.data_ptr(), k.data_ptr(), v.data_ptr(),
         _native.ptr(ws), 0 if ws is None else ws.numel(), stream)
-    _native.check(status, "mqk_fused_qkv_rope_bf16")
+    _native.check(status, entry)
     return q, k, v
 
 
