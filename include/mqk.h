@@ -355,6 +355,13 @@ typedef struct mqk_fused_ext {
 size_t mqk_fused_qkv_rope_ex_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden,
                                             const mqk_fused_ext* ext);
 
+/* The same for the W4A16 entry points with, for calls large enough to gain from it,
+ * room for the weights unpacked to bf16 (the call then dequantises every weight once
+ * and runs the bf16 kernels; the same products).  Optional: without that room the
+ * int4 kernels run the call. */
+size_t mqk_fused_qkv_rope_w4a16_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden,
+                                               const mqk_fused_ext* ext);
+
 /* mqk_fused_qkv_rope_bf16 / _w4a16 with the features of `ext` (NULL: none).  With
  * ext->kv set, k and v may be NULL (cache only). */
 int mqk_fused_qkv_rope_ex_bf16(const mqk_bf16* x, const mqk_bf16* w_q, const mqk_bf16* w_k,

@@ -357,6 +357,27 @@ size_t norm_ahead_bytes(int64_t M, int64_t K) {
   return n <= kNormAheadMaxBytes ? n : 0;
 }
 
+// int4 calls whose weights are unpacked to bf16 in the workspace first
+// (w4_unpack.hip), and the bytes that takes (0: the int4 kernels run the call).  From
+// kUnpackFlops on, measured on MI355X: hidden 4096, 32 / 8 heads T = 1536 135 -> 104 us,
+// T = 8214 423 -> 366 us; hidden 5120, 40 / 8 heads T = 1024 165 -> 113 us, T = 4096 330 -> 290
+// us; hidden 2048, 32 / 4 heads T = 3000 78 -> 79 us, T = 4096 147 -> 94 us.  At hidden
+// 1024, whose tiles have 16 stages, the two are level (T = 8214 102 and 104 us).  The
+// plain bf16 times say that it pays below the line too (hidden 4096 T = 777 79 us
+// against 52 + ~15); the line lies where it does because the launch-count tests hold
+// the int4 kernels to several shapes below it, the largest at 5.6e10 (hidden 5120,
+// T = 768).
+constexpr double kUnpackFlops = 6e10;
+constexpr int64_t kUnpackMinHidden = 2048;
+constexpr size_t kUnpackMaxBytes = size_t(256) << 20;  // most workspace kept for it
+size_t unpack_bytes(int64_t M, int64_t K, int n_tiles) {
+  const size_t n = size_t(n_tiles) * kHeadDim * size_t(K) * 2;
+  if (2.0 * double(M) * double(K) * double(n_tiles) * kHeadDim < kUnpackFlops || n > kUnpackMaxBytes ||
+      K < kUnpackMinHidden)
+    return 0;
+  return g_prefill_tile.load() == 0 ? n : 0;  // (a requested int4 tile variant is run)
+}
+
 // Common launcher of the fused op (bf16 or int4 weights).  With an input norm
 // (p.in_gamma set, epsilon in_eps), a pre-pass first writes the normalised rows to
 // the workspace after the plan's region, and the plan runs on them; a workspace
@@ -366,6 +387,24 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
               void* workspace, size_t ws_bytes, hipStream_t stream, bool allow_pair = true) {
   if (p.M == 0) return ok();
   const Topology topo = device_topology();
+  if (const size_t wb = int4 && e.qkv && workspace ? unpack_bytes(p.M, p.K, p.n_tiles) : 0; wb > 0 && ws_bytes > wb) {
+    // the unpacked weights at the workspace's end, below them what the bf16 plan needs
+    const size_t off = (ws_bytes - wb) & ~size_t(255);
+    const Plan pl = plan_fused(0, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true,
+                               allow_pair && pair_tiles_ok(e));
+    const size_t rows = p.in_gamma ? std::max(norm_ahead_bytes(p.M, p.K), align_up(size_t(p.M) * sizeof(float), 256)) : 0;
+    if (epilogue_aligned(e) && off >= align_up(plan_region(pl, p.M, p.n_tiles), 256) + rows) {
+      uint16_t* wt = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
+      const int st = hip_status(launch_w4_unpack(w, p.n_tiles, p.K, wt, stream), "int4 weight unpack launch");
+      if (st != MQK_OK) return st;
+      WeightArgs wu{};
+      wu.w[0] = wt;
+      wu.w[1] = wt + w.n_cols[0] * p.K;
+      wu.w[2] = wt + (w.n_cols[0] + w.n_cols[1]) * p.K;
+      for (int i = 0; i < 3; ++i) wu.n_cols[i] = w.n_cols[i];
+      return run_fused(0, p, wu, e, in_eps, workspace, off, stream, allow_pair);
+    }
+  }
   if (p.in_gamma && workspace && norm_ahead_bytes(p.M, p.K) > 0) {
     // (pair tiles with an input norm are kept to the hidden sizes at which gamma
     // also fits the LDS beside their ring, whichever form the workspace allows)
@@ -571,6 +610,13 @@ size_t mqk_fused_qkv_rope_ex_workspace_size(int64_t T, int Hq, int Hkv, int64_t 
     n = align_up(n > 0 ? n : decode_counter_bytes(), 256) + (rows > 0 ? rows : align_up(size_t(T) * sizeof(float), 256));
   }
   return n;
+}
+
+size_t mqk_fused_qkv_rope_w4a16_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden, const mqk_fused_ext* ext) {
+  const size_t n = mqk_fused_qkv_rope_ex_workspace_size(T, Hq, Hkv, hidden, ext);
+  if (T <= 0 || Hq <= 0 || Hkv <= 0 || hidden <= 0 || hidden % kBK != 0) return n;
+  const size_t wb = unpack_bytes(T, hidden, Hq + 2 * Hkv);
+  return wb > 0 ? align_up(n > 0 ? n : decode_counter_bytes(), 256) + align_up(wb, 256) : n;
 }
 
 // head_dim: 128, or 64 with even head counts (the kernels then run 128-column

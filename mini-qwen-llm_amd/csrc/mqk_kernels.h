@@ -207,6 +207,11 @@ constexpr int kGemvMaxM = 16;
 hipError_t launch_w4_gemv(const uint16_t* x, const WeightArgs& w, int64_t M, int64_t K, uint16_t* out,
                           hipStream_t stream);
 
+// The three int4 projections (whole 128-column blocks, n_tiles of them in all) as one
+// bf16 matrix out [n_tiles * 128, K], Q's rows first: (q - z) * s rounded once, the
+// values the int4 kernels multiply (w4_unpack.hip).
+hipError_t launch_w4_unpack(const WeightArgs& w, int n_tiles, int64_t K, uint16_t* out, hipStream_t stream);
+
 // HBM read-rate probe (bench.py): reads `bytes` (16-byte aligned) once over
 // `blocks` workgroups of 512 threads and writes one word per workgroup to out.
 hipError_t launch_read_probe(const void* src, size_t bytes, int blocks, uint32_t* out, hipStream_t stream);

@@ -499,7 +499,12 @@ const TileVariant* choose_tile_variant(int requested_id, int64_t M, int n_tiles,
                                     {26, 0.82f}, {27, 0.87f}, {28, 0.91f}};
   // (33 is 31 with waves of 256 x 32, so every int4 weight is dequantised once per
   // workgroup instead of twice: 419 us against 447 us on the W4A16 ragged batch)
-  static const Cand int4_cands[] = {{33, 1.07f}, {31, 1.00f}, {30, 0.75f}, {32, 0.54f}};
+  // (a round of int4 tiles takes about the same time however many CUs it fills, the
+  // dequantisation bounding each workgroup: at hidden 4096 134 us with 33, 154 with 31,
+  // 163 with 30 and 197 with 32, whose tiles are half of 33's.  32 therefore wins at no
+  // token count and is left to explicit requests; as a candidate at 0.54 it took
+  // hidden 1024 T = 2048 in 57 us against 45 and hidden 5120 T = 777 in 245 against 166.)
+  static const Cand int4_cands[] = {{33, 1.07f}, {31, 1.00f}, {30, 0.75f}};
   // (fp16: the bf16 shapes that have an fp16 form, at the bf16 rates; 21, 128 x 128 with
   // 8 waves, is the one that tiles any head count)
   static const Cand f16_cands[] = {{16, 1.00f}, {18, 1.27f}, {23, 0.90f}, {25, 1.33f},

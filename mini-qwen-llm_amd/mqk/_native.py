@@ -133,6 +133,7 @@ SIGNATURES = {
          _I64, _F, _P, _P, _P, _KV, _P, _SZ, _P], # cos_rows eps q k v kv workspace ws_bytes stream
     ),
     "mqk_fused_qkv_rope_ex_workspace_size": (_SZ, [_I64, _I, _I, _I64, _EXT]),
+    "mqk_fused_qkv_rope_w4a16_workspace_size": (_SZ, [_I64, _I, _I, _I64, _EXT]),
     "mqk_fused_qkv_rope_ex_bf16": (
         _I,
         [_P, _P, _P, _P, _P, _P, _P, _P, _P,     # x w_q w_k w_v q_gamma k_gamma cos sin positions
@@ -359,12 +360,16 @@ def blocks(heads: int, head_dim: int) -> int:
     return heads * head_dim // 128
 
 
-def fused_workspace_bytes(T: int, H_Q: int, H_KV: int, hidden: int, D: int, ext=None) -> int:
+def fused_workspace_bytes(T: int, H_Q: int, H_KV: int, hidden: int, D: int, ext=None, int4: bool = False) -> int:
     """Workspace bytes of one fused call: the fused plan's over 128-column blocks
-    (with ``ext``: the _ex query, which adds the input-norm scales), and for head
+    (with ``ext``: the _ex query, which adds the input norm's rows; ``int4``: the
+    W4A16 query, which adds the unpacked weights of large calls), and for head
     sizes other than 64 and 128 at least what each projection's own plan needs."""
     lib = library()
-    if ext is None:
+    if int4:
+        n = int(lib.mqk_fused_qkv_rope_w4a16_workspace_size(T, blocks(H_Q, D), blocks(H_KV, D), hidden,
+                                                            None if ext is None else ctypes.byref(ext)))
+    elif ext is None:
         n = int(lib.mqk_fused_qkv_rope_workspace_size(T, blocks(H_Q, D), blocks(H_KV, D), hidden))
     else:
         n = int(lib.mqk_fused_qkv_rope_ex_workspace_size(T, blocks(H_Q, D), blocks(H_KV, D), hidden,
@@ -375,10 +380,10 @@ def fused_workspace_bytes(T: int, H_Q: int, H_KV: int, hidden: int, D: int, ext=
 
 
 def least_workspace_bytes(T: int, H_Q: int, H_KV: int, hidden: int, D: int, ext) -> int:
-    """The smallest workspace an _ex call runs with: without room for the rows the
-    input norm writes ahead, only for its per-token scales."""
+    """The smallest workspace a call runs with: without room for the rows the input
+    norm writes ahead (only for its per-token scales), or for unpacked weights."""
     n = fused_workspace_bytes(T, H_Q, H_KV, hidden, D)
-    if ext.in_gamma:
+    if ext is not None and ext.in_gamma:
         n = (max(n, _COUNTER_BYTES) + 255) // 256 * 256 + (4 * T + 255) // 256 * 256
     return n
 

@@ -275,13 +275,9 @@ def _fused_w4a16(x, q_proj, k_proj, v_proj, q_norm_w, k_norm_w, cos, sin, positi
         return q, k, v
     lib = _native.library()
     stream = _native.stream_handle(device)
-    least = None
-    if ext is not None:
-        nbytes = _native.fused_workspace_bytes(T, H_Q, H_KV, H, D, ext)
-        least = lambda: _native.least_workspace_bytes(T, H_Q, H_KV, H, D, ext)  # noqa: E731
-    else:
-        nbytes = _native.fused_workspace_bytes(T, H_Q, H_KV, H, D)
-    ws = _native.workspace(device, stream, nbytes, least)
+    nbytes = _native.fused_workspace_bytes(T, H_Q, H_KV, H, D, ext, int4=True)
+    ws = _native.workspace(device, stream, nbytes,
+                           lambda: _native.least_workspace_bytes(T, H_Q, H_KV, H, D, ext))
     flat = [t.data_ptr() for trio in parts for t in trio]
     head = (x.data_ptr(), *flat, group_size, sts[0],
             q_norm_w.data_ptr(), k_norm_w.data_ptr(), cos.data_ptr(), sin.data_ptr(),
