@@ -26,7 +26,8 @@ CSRC = Path(__file__).resolve().parent
 PKG = CSRC.parent / "mqk"
 OUT = PKG / "libmqk.so"
 BUILD_DIR = CSRC.parent / "_build"
-SOURCES = ["qkv_tile.hip", "qkv_tile_dma.hip", "qkv_decode.hip", "norm_rope.hip", "input_norm.hip", "qkv_f32.hip",
+SOURCES = ["qkv_tile.hip", "qkv_tile_dma.hip", "qkv_decode.hip", "qkv_decode_multi.hip", "qkv_decode_w4.hip",
+           "qkv_decode_w4_multi.hip", "qkv_decode_f16.hip", "norm_rope.hip", "input_norm.hip", "qkv_f32.hip",
            "w4_gemv.hip", "w4_unpack.hip", "read_probe.hip", "mqk_api.hip"]
 # No kernel may use scratch memory (register spills, or an array the compiler
 # could not keep in registers): the compiler's resource-usage remarks of every

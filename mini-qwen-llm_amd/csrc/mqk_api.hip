@@ -163,15 +163,12 @@ struct Plan {
 //   256 x 256 (hidden 1024 / 2048 / 5120 with 32 / 40 / 56 heads, T = 128 .. 1536,
 //     2 to 8 splits; rms error 1.5 us): 12.6 us, 1.6 us per stage of
 //     ceil(stages / splits), 0.195 us per MB, 0.35 us per unit.
-// (The 256 x 256 split kernel has no input-norm form: with the norm's registers it
-// would spill.)
-int plan_tile_split(int64_t M, int64_t K, int n_tiles, const Topology& topo, bool in_norm, const TileVariant*& v,
-                    double& us) {
+int plan_tile_split(int64_t M, int64_t K, int n_tiles, const Topology& topo, const TileVariant*& v, double& us) {
   v = nullptr;
   us = 1e30;
   const int64_t req = g_tile_ksplit.load();
   if (req == 0 || g_prefill_tile.load() != 0) return 0;
-  const int id = n_tiles % 3 == 0 ? 16 : (n_tiles % 2 == 0 && !in_norm ? 18 : 0);
+  const int id = n_tiles % 3 == 0 ? 16 : (n_tiles % 2 == 0 ? 18 : 0);
   if (id == 0) return 0;
   for (int i = 0; i < tile_variant_count(); ++i)
     if (tile_variant(i)->id == id) v = tile_variant(i);
@@ -199,14 +196,19 @@ int plan_tile_split(int64_t M, int64_t K, int n_tiles, const Topology& topo, boo
   return best;
 }
 
+// in_norm: the kernels normalise x themselves (a workspace without room for the
+// normalised rows): whole-head and single-head tiles only.  allow_decode false: a
+// workspace without room for the decode kernel's partials (fp16 only; the other types'
+// entry points require it).
 Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const Topology& topo,
                 bool allow_blocks = true, bool in_norm = false, bool allow_split = true, bool allow_pair = false,
-                int half = 0) {
+                int half = 0, bool allow_decode = true) {
+  if (in_norm) allow_decode = allow_blocks = allow_split = allow_pair = false;
   allow_pair = allow_pair && !int4 && aligned && g_pair_tiles.load() != 0;
   Plan pl;
   const int64_t cus = topo.cus;
-  if (half) allow_blocks = allow_split = false;  // (fp16 runs on the tile kernels only)
-  if (use_decode(M) && aligned && !half) {
+  if (half) allow_blocks = allow_split = false;  // (fp16: the one-block decode kernel and the tiles)
+  if (use_decode(M) && aligned && allow_decode) {
     pl.splits = decode_splits_for(M, K, n_tiles, int(g_decode_splits.load()), topo.cus, topo.xcds);
     if (pl.splits > 0) {
       pl.tail = M;
@@ -233,7 +235,7 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
   const int64_t nblk = (M + 63) / 64;
   const int blk_splits = decode_splits_for(64, K, n_tiles, int(g_decode_splits.load()), topo.cus, topo.xcds);
   const int64_t per_launch = std::max<int64_t>(
-      1, std::min<int64_t>(g_decode_passes.load(), decode_max_blocks(n_tiles, K, blk_splits, int4 && in_norm)));
+      1, std::min<int64_t>(g_decode_passes.load(), decode_max_blocks(n_tiles, K, blk_splits)));
   const int64_t launches = (nblk + per_launch - 1) / per_launch;
   const double w_bytes = double(n_tiles) * kHeadDim * double(K) * (int4 ? 0.5 : 2.0);
   // (int4's first block is bound by the 64-k tiles each split dequantises and
@@ -250,7 +252,7 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
   // per-tile launch and the decode blocks
   const TileVariant* sv = nullptr;
   double split_us = 1e30;
-  const int ksplit = (!int4 && aligned && allow_split && M > 64) ? plan_tile_split(M, K, n_tiles, topo, in_norm, sv, split_us) : 0;
+  const int ksplit = (!int4 && aligned && allow_split && M > 64) ? plan_tile_split(M, K, n_tiles, topo, sv, split_us) : 0;
   // One round of single-head tiles: 64 x 128 while ceil(M/64) x heads fit the CUs,
   // else 128 x 128 with 8 waves while ceil(M/128) x heads do.  Neither needs a
   // partial exchange.  Fitted on MI355X over hidden 2048 / 4096 / 5120 (40 / 48 / 56
@@ -261,7 +263,7 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
   //   launch, e.g. hidden 5120 at T = 384 / 512: 98 us against 119 / 158).
   const TileVariant* hv = nullptr;
   double head_us = 1e30;
-  if (aligned && (M > 64 || half) && g_prefill_tile.load() == 0 && g_head_tiles.load() != 0) {
+  if (aligned && (M > 64 || !allow_decode) && g_prefill_tile.load() == 0 && g_head_tiles.load() != 0) {
     const int64_t t64 = (M + 63) / 64 * n_tiles, t128 = (M + 127) / 128 * n_tiles;
     const double stages = double(K / 64);
     const bool one64 = t64 <= cus, one128 = t128 <= cus;
@@ -285,8 +287,7 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
     for (int i = 0; i < tile_variant_count(); ++i)
       if (tile_variant(i)->id == 26) pv = tile_variant(i);
     const int64_t wgs = pv ? tile_count(*pv, M, n_tiles) : 0;
-    if (pv && 2 * wgs > cus && wgs <= cus && wgs / 2 <= kSplitMaxTiles &&
-        !(in_norm && tile_dma_lds_bytes(26) + K * 2 > 160 * 1024)) {
+    if (pv && 2 * wgs > cus && wgs <= cus && wgs / 2 <= kSplitMaxTiles) {
       pair_us = 15.0 + double(K / 64) * (0.465 + 0.001 * double(wgs));
     } else {
       pv = nullptr;
@@ -317,7 +318,7 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
     return pl;
   }
   pl.v = choose_tile_variant(int(g_prefill_tile.load()), M, n_tiles, int4, topo.cus, allow_pair, half);
-  if (half || !pl.v || !g_tail_split.load() || !aligned || M <= 64) return pl;
+  if (!allow_decode || !pl.v || !g_tail_split.load() || !aligned || M <= 64) return pl;
   const int64_t r = M % pl.v->bm;
   if (r == 0 || r > 64 || !use_decode(r)) return pl;
   const int64_t rounds_all = (tile_count(*pl.v, M, n_tiles) + cus - 1) / cus;
@@ -435,16 +436,13 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
   // bytes the plan needs: the decode (or split-tile) region, then (input norm) the per-token scales
   const size_t scale_bytes = p.in_gamma ? align_up(size_t(p.M) * sizeof(float), 256) : 0;
   auto fits = [&](size_t b) { return workspace && ws_bytes >= align_up(b, 256) + scale_bytes; };
-  const bool split_ok = epilogue_aligned(e) && !(p.in_gamma && pl.v && tile_dma_lds_bytes(pl.v->id) + p.K * 2 > 160 * 1024);
-  if (pl.ksplit > 0 && (!fits(base) || !split_ok)) {
+  if (pl.ksplit > 0 && (!fits(base) || !epilogue_aligned(e))) {
     // a workspace sized without the split-K tile launch (or operands it cannot take): plan without it
     pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, false, pair_ok, p.half);
     base = region(pl);
   }
-  if (pl.v && is_pair_variant(pl.v->id) &&
-      (!fits(base) || (p.in_gamma && tile_dma_lds_bytes(pl.v->id) + p.K * 2 > 160 * 1024))) {
-    // a workspace sized without the pair tiles' exchange area, or an input norm whose
-    // gamma does not fit the LDS beside their ring: plan without them
+  if (pl.v && is_pair_variant(pl.v->id) && !fits(base)) {
+    // a workspace sized without the pair tiles' exchange area: plan without them
     pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, false, false, p.half);
     base = region(pl);
   }
@@ -455,6 +453,11 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
   if (!pl.v && p.M > 64 && !fits(base)) {
     // decode blocks planned, but a workspace sized without them: the tile kernel
     pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, false, p.in_gamma != nullptr, false);
+    base = region(pl);
+  }
+  if (p.half && !pl.v && !fits(base)) {
+    // fp16 without a workspace for the decode kernel: tiles
+    pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, false, false, false, false, 1, false);
     base = region(pl);
   }
   if (pl.v && pl.splits > 0 && !fits(base)) {
@@ -544,10 +547,9 @@ const char* mqk_last_error_detail(void) { return g_detail; }
 // Workspace bytes run_fused's plan of `tiles` 128-column blocks needs (before
 // any input-norm scales): a plain GEMM (bf16 or int4 weights, no pair tiles), or
 // with allow_pair the q/k/v launch of the generic head sizes.
-static size_t plan_bytes(int int4, int64_t M, int64_t K, int tiles, const Topology& topo, bool in_norm,
-                         bool allow_pair) {
+static size_t plan_bytes(int int4, int64_t M, int64_t K, int tiles, const Topology& topo, bool allow_pair) {
   if (tiles > kMaxTiles) return ~size_t(0);
-  const Plan pl = plan_fused(int4, M, K, tiles, true, topo, true, in_norm, true, allow_pair);
+  const Plan pl = plan_fused(int4, M, K, tiles, true, topo, true, false, true, allow_pair);
   size_t n = 0;
   if (pl.splits > 0) n = std::max(n, decode_workspace_bytes(tiles, pl.splits, pl.passes));
   if (pl.ksplit > 0) n = std::max(n, kDecodeCounterBytes + tile_split_part_bytes(pl.v->id, M, tiles, pl.ksplit));
@@ -557,7 +559,7 @@ static size_t plan_bytes(int int4, int64_t M, int64_t K, int tiles, const Topolo
 
 static size_t plain_plan_bytes(int int4, int64_t M, int64_t K, int tiles, const Topology& topo) {
   if (int4 && M <= g_gemv_max_m.load()) return 0;  // the column-parallel kernel needs none
-  return plan_bytes(int4, M, K, tiles, topo, false, false);
+  return plan_bytes(int4, M, K, tiles, topo, false);
 }
 
 size_t mqk_fused_qkv_rope_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden) {
@@ -586,12 +588,11 @@ size_t mqk_fused_qkv_rope_workspace_size_hd(int64_t T, int Hq, int Hkv, int64_t 
   if ((int64_t(Hq) * head_dim) % kHeadDim == 0 && (int64_t(Hkv) * head_dim) % kHeadDim == 0)
     for (int int4 = 0; int4 < 2; ++int4) {
       const int tiles = int((int64_t(Hq) + 2 * Hkv) * head_dim / kHeadDim);
-      const size_t m = plan_bytes(int4, T, hidden, tiles, topo, false, true);
-      if (m != ~size_t(0)) n = std::max(n, m);
-      // (with the fused input RMSNorm: that plan, then the per-token scales)
-      const size_t mn = plan_bytes(int4, T, hidden, tiles, topo, true, true);
-      if (mn != ~size_t(0))
-        n = std::max(n, align_up(mn > 0 ? mn : decode_counter_bytes(), 256) + align_up(size_t(T) * sizeof(float), 256));
+      const size_t m = plan_bytes(int4, T, hidden, tiles, topo, true);
+      // (with the fused input RMSNorm: that plan, then the normalised rows or the scales)
+      if (m != ~size_t(0))
+        n = std::max(n, align_up(m > 0 ? m : decode_counter_bytes(), 256) +
+                            std::max(norm_ahead_bytes(T, hidden), align_up(size_t(T) * sizeof(float), 256)));
     }
   for (int int4 = 0; int4 < 2; ++int4)
     for (int h : {Hq, Hkv}) {
@@ -769,11 +770,10 @@ static int fused_bf16_any_d(const mqk_bf16* x, const mqk_bf16* w_q, const mqk_bf
     // as projected (qkv 2), when the workspace holds what that plan needs
     const bool in_norm = ext && ext->in_gamma;
     const int tiles = int((nq + 2 * nkv) / kHeadDim);
-    const size_t need = plan_bytes(0, T, hidden, tiles, topo, in_norm, true);
-    const size_t scales = in_norm ? align_up(size_t(T) * sizeof(float), 256) : 0;
-    const bool fits = need != ~size_t(0) &&
-                      ((need == 0 && !in_norm) ||
-                       (workspace && align_up(need > 0 ? need : decode_counter_bytes(), 256) + scales <= ws_bytes));
+    // (with the input norm the launch takes any workspace that holds its scales)
+    const size_t need = in_norm ? align_up(decode_counter_bytes(), 256) + align_up(size_t(T) * sizeof(float), 256)
+                                : plan_bytes(0, T, hidden, tiles, topo, true);
+    const bool fits = tiles <= kMaxTiles && need != ~size_t(0) && (need == 0 || (workspace && need <= ws_bytes));
     if (fits) {
       ProblemArgs pr{x, T, hidden, tiles};
       pr.in_gamma = in_norm ? ext->in_gamma : nullptr;
@@ -1279,11 +1279,9 @@ static int fused_w4a16_impl(const mqk_bf16* x, const int32_t* qw_q, const void* 
             MQK_OK)
           return st;
       const int tiles = int((nq + 2 * nkv) / kHeadDim);
-      const size_t need = plan_bytes(1, T, hidden, tiles, topo, in_norm, true);
-      const size_t scales = in_norm ? align_up(size_t(T) * sizeof(float), 256) : 0;
-      if (need != ~size_t(0) &&
-          ((need == 0 && !in_norm) ||
-           (workspace && align_up(need > 0 ? need : decode_counter_bytes(), 256) + scales <= ws_bytes))) {
+      const size_t need = in_norm ? align_up(decode_counter_bytes(), 256) + align_up(size_t(T) * sizeof(float), 256)
+                                  : plan_bytes(1, T, hidden, tiles, topo, true);
+      if (tiles <= kMaxTiles && need != ~size_t(0) && (need == 0 || (workspace && need <= ws_bytes))) {
         ProblemArgs pr{x, T, hidden, tiles};
         pr.in_gamma = in_norm ? ext->in_gamma : nullptr;
         WeightArgs w{};

@@ -171,7 +171,7 @@ size_t decode_workspace_bytes(int n_tiles, int splits, int blocks = 1);
 // Most 64-row blocks one decode launch may cover with this many heads and splits
 // (one arrival counter per (head, block) in the workspace's counter region; one
 // block when a split's k range is too long to hold its weights in registers).
-int decode_max_blocks(int n_tiles, int64_t K, int splits, bool int4_norm);
+int decode_max_blocks(int n_tiles, int64_t K, int splits);
 // The decode kernel's counters open every workspace: one arrival counter per
 // head (kDecodeMaxHeads), then a statistics line whose first word counts the
 // heads finished on the recompute path (a split ran on an unexpected XCD), then
@@ -188,7 +188,8 @@ size_t decode_counter_bytes();
 // The split-K decode kernel on the launch's p.M rows: ceil(M / 64) <=
 // decode_max_blocks(n_tiles) blocks of 64 rows share one stream of the weights;
 // the workspace holds decode_workspace_bytes(n_tiles, splits, blocks).  With
-// e.qkv == 0 it writes the plain product to e.out ([M, N], N = 128 * n_tiles).
+// e.qkv == 0 it writes the plain product to e.out ([M, N], N = 128 * n_tiles).  No
+// input norm (x is normalised ahead); fp16 (p.half) for one block only.
 hipError_t launch_decode(int int4, const ProblemArgs& p, const WeightArgs& w, const EpilogueArgs& e,
                          int splits, void* workspace, hipStream_t stream);
 

@@ -850,7 +850,7 @@ tile_dma_f16_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, int group_m, Pa
 
 // The split-K launch of the pipelined kernel (a separate kernel, so that the
 // one-workgroup-per-tile kernel above keeps its own register allocation).
-template <int BM, int NH, int WM, int WN, int NS, int SBK, bool INORM>
+template <int BM, int NH, int WM, int WN, int NS, int SBK>
 __global__ void __launch_bounds__(WM* WN * 64)
 tile_dma_split_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, TileSplit sp) {
   using S = DmaShape<BM, NH, WM, WN, NS, SBK>;
@@ -917,23 +917,6 @@ tile_dma_split_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, TileSplit sp)
     }
     dst_off[i] = uint32_t(row0 * kRowBytes);
   }
-  // input RMSNorm: scale of the x row and k offset of the chunk each of this
-  // lane's x loads brings in (load i < kALoads, row0 + lane / chunks, slot lane % chunks)
-  constexpr bool in_norm = INORM;  // (p.in_gamma != nullptr: a template switch keeps its registers out of the plain kernel)
-  float a_scale[S::kALoads];
-  int a_koff[S::kALoads];
-#pragma unroll
-  for (int i = 0; i < S::kALoads; ++i) {
-    const int row = S::kRowsPerLoad * (wave + i * S::kWaves) + lane / S::kChunks;
-    int64_t grow = m0 + row;
-    grow = grow < p.M ? grow : p.M - 1;
-    a_scale[i] = in_norm ? p.in_scale[grow] : 1.f;
-    a_koff[i] = stage_slot<SBK>(row, lane % S::kChunks) * 8;
-  }
-  if (in_norm) {
-    stage_gamma<S::kThreads>(p);
-    __syncthreads();
-  }
   // stage j of a k range starting at stage kt0 goes to ring slot j % NS
   auto issue = [&](int kt0, int j) {
     const uint32_t base = lds0 + uint32_t((j % NS) * S::kStageBytes);
@@ -959,13 +942,6 @@ tile_dma_split_kernel(ProblemArgs p, WeightArgs w, EpilogueArgs e, TileSplit sp)
     for (int kt = 0; kt < nkt; ++kt) {
       const int ahead = min(NS - 2, nkt - 1 - kt);  // stages already issued after kt
       wait_stage<NS, S::kLoadsPerWave>(ahead);
-      if (in_norm) {  // this wave's x chunks of stage kt have landed: normalise them in place
-#pragma unroll
-        for (int i = 0; i < S::kALoads; ++i)
-          norm_chunk(smem + (kt % NS) * S::kStageBytes + dst_off[i] + lane * 16,
-                     int64_t(kt0 + kt) * SBK + a_koff[i], a_scale[i]);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      }
       barrier();
       if (kt + NS - 1 < nkt) issue(kt0, kt + NS - 1);
       const unsigned char* st = smem + (kt % NS) * S::kStageBytes;
@@ -1255,9 +1231,9 @@ hipError_t launch_dma_split(const ProblemArgs& p, const WeightArgs& w, const Epi
   const int tiles = n_mt * (p.n_tiles / NH);
   const int X = p.xcds > 0 ? p.xcds : 1;
   const int tpx = (tiles + X - 1) / X;
-  const size_t dyn = p.in_gamma ? size_t(p.K) * 2 : 0;
-  // (p.xcds <= 8: the arrival word's XCD sums hold x < 8)
-  if (S::kLdsBytes + dyn > 160 * 1024 || ksplit < 2 || ksplit > 16 || tiles > kSplitMaxTiles || p.xcds > 8 ||
+  // (no input-norm form: x is normalised ahead.  p.xcds <= 8: the arrival word's XCD sums
+  // hold x < 8)
+  if (p.in_gamma || ksplit < 2 || ksplit > 16 || tiles > kSplitMaxTiles || p.xcds > 8 ||
       p.K / SBK < ksplit)
     return hipErrorInvalidValue;
   TileSplit sp;
@@ -1266,16 +1242,8 @@ hipError_t launch_dma_split(const ProblemArgs& p, const WeightArgs& w, const Epi
   sp.max_spins = max_spins;
   sp.counters = static_cast<uint32_t*>(workspace);
   sp.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + kDecodeCounterBytes);
-  if (p.in_gamma) {
-    // (no input-norm form of the 256-row tiles: its registers would spill)
-    if constexpr (BM > 128) return hipErrorInvalidValue;
-    else
-      hipLaunchKernelGGL((tile_dma_split_kernel<BM, NH, WM, WN, NS, SBK, true>), dim3(X * ksplit * tpx),
-                         dim3(S::kThreads), dyn, stream, p, w, e, sp);
-  } else {
-    hipLaunchKernelGGL((tile_dma_split_kernel<BM, NH, WM, WN, NS, SBK, false>), dim3(X * ksplit * tpx),
-                       dim3(S::kThreads), dyn, stream, p, w, e, sp);
-  }
+  hipLaunchKernelGGL((tile_dma_split_kernel<BM, NH, WM, WN, NS, SBK>), dim3(X * ksplit * tpx), dim3(S::kThreads), 0,
+                     stream, p, w, e, sp);
   return hipGetLastError();
 }
 
