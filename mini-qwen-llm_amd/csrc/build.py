@@ -6,7 +6,8 @@
                                                           # newer than their object
 
 Every translation unit is compiled in parallel, then linked into
-``mini-qwen-llm_amd/mqk/libmqk.so`` (the location the ``mqk`` package loads).
+``mini-qwen-llm_amd/mqk/libmqk.so`` (the location the ``mqk`` package loads);
+``front.cpp``, the package's CPython extension, becomes ``mqk/_front<suffix>``.
 The compile flags switch off packed-fp32 instruction selection for the device
 pass (``-target-feature -packed-fp32-ops``); hipcc's host pass prints a
 harmless "not a recognized feature" warning for it.
@@ -20,11 +21,14 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 CSRC = Path(__file__).resolve().parent
 PKG = CSRC.parent / "mqk"
 OUT = PKG / "libmqk.so"
+FRONT_SRC = CSRC / "front.cpp"
+FRONT = PKG / f"_front{sysconfig.get_config_var('EXT_SUFFIX')}"
 BUILD_DIR = CSRC.parent / "_build"
 SOURCES = ["qkv_tile.hip", "qkv_tile_dma.hip", "qkv_decode.hip", "qkv_decode_multi.hip", "qkv_decode_w4.hip",
            "qkv_decode_w4_multi.hip", "qkv_decode_f16.hip", "norm_rope.hip", "input_norm.hip", "qkv_f32.hip",
@@ -97,16 +101,41 @@ def _compile(src: str, verbose: bool, incremental: bool = False) -> Path:
     if check:
         bad = _scratch_kernels(out)
         if bad:
+            obj.unlink(missing_ok=True)  # (an incremental build must not take it as up to date)
             raise RuntimeError(f"{src}: kernels use scratch memory (register spills): " + "; ".join(bad))
     if msg and verbose:
         print(msg)
     return obj
 
 
+def _build_front(verbose: bool, incremental: bool) -> None:
+    """The CPython extension (host code only, against the installed torch)."""
+    if incremental and FRONT.exists() and all(
+            d.stat().st_mtime < FRONT.stat().st_mtime
+            for d in (FRONT_SRC, CSRC.parent.parent / "include" / "mqk.h", Path(__file__))):
+        return
+    import torch
+    from torch.utils.cpp_extension import include_paths
+    lib = Path(torch.__file__).parent / "lib"
+    tmp = FRONT.with_suffix(".tmp")
+    cmd = [os.environ.get("CXX", "g++"), "-std=c++17", "-O2", "-fPIC", "-Wall", "-shared",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", str(FRONT_SRC), "-o", str(tmp),
+           "-I" + sysconfig.get_paths()["include"], *(a for p in include_paths() for a in ("-isystem", p)),
+           f"-L{lib}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-ldl"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"front.cpp failed:\n{res.stdout}{res.stderr}")
+    os.replace(tmp, FRONT)
+
+
 def build(verbose: bool = False, incremental: bool = False) -> Path:
     BUILD_DIR.mkdir(exist_ok=True)
-    with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES), os.cpu_count() or 1)) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES) + 1, os.cpu_count() or 1)) as ex:
+        front = ex.submit(_build_front, verbose, incremental)
         objs = list(ex.map(lambda s: _compile(s, verbose, incremental), SOURCES))
+        front.result()
     tmp = OUT.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     if verbose:

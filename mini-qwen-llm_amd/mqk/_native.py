@@ -187,6 +187,37 @@ def library() -> ctypes.CDLL:
     return _lib
 
 
+# The C++ form of the entry points' checks, allocations and call (csrc/front.cpp) for
+# ordinary calls; None until bound, and for good where it was not built (the Python
+# code runs every call then, on the same kernels).
+_front = None
+_front_absent = False
+
+
+def front():
+    """The bound ``mqk._front`` extension, or None (not built, or the library is not
+    there to bind: the Python path raises for that)."""
+    global _front, _front_absent
+    if _front is not None or _front_absent:
+        return _front
+    try:
+        lib = library()
+    except MqkNativeError:
+        return None
+    with _lock:
+        if _front is None and not _front_absent:
+            try:
+                from . import _front as ext
+            except ImportError:
+                ext = None
+            if ext is None or _raw_stream is None:
+                _front_absent = True
+            else:
+                ext.bind(lib._handle, _workspaces, _raw_stream, torch.nn.Parameter)
+                _front = ext
+    return _front
+
+
 def call(device: torch.device, fn, *args) -> int:
     """Run one native entry point with ``device`` as the current HIP device.
 

@@ -100,6 +100,10 @@ def _no_bytes() -> int:
     return 0
 
 
+_ENTRIES = {torch.bfloat16: "mqk_fused_qkv_rope_bf16", torch.float16: "mqk_fused_qkv_rope_f16_ws",
+            torch.float32: "mqk_fused_qkv_rope_f32"}
+
+
 def fused_qkv_rope(
     x: torch.Tensor,
     w_q: torch.Tensor,
@@ -112,6 +116,13 @@ def fused_qkv_rope(
     positions: Optional[torch.Tensor] = None,
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Fused QKV projection + QK-Norm + RoPE; see the module docstring."""
+    front = _native._front or _native.front()
+    if front is not None:  # (an ordinary call in C++; None: one for the code below)
+        out = front.fused(x, w_q, w_k, w_v, q_norm_w, k_norm_w, cos, sin, positions)
+        if out is not None:
+            if type(out) is int:
+                _native.check(out, _ENTRIES[x.dtype])
+            return out
     B, S, H = x.shape
     D = q_norm_w.shape[0]
     H_Q = w_q.shape[0] // D
@@ -228,6 +239,14 @@ def fused_qkv_rope_paged(
     (unless ``return_kv`` is False) and once to their cache slot.  Returns
     ``(q, k, v)``, with ``k``/``v`` None when ``return_kv`` is False.
     """
+    front = _native._front or _native.front()
+    if front is not None and k_cache is not None:
+        out = front.fused_ex(x, w_q, w_k, w_v, q_norm_w, k_norm_w, cos, sin, positions, None, None, None, EPS, k_cache,
+                             v_cache, block_table, kv_seq, kv_pos, return_kv)
+        if out is not None:
+            if type(out) is int:
+                _native.check(out, "mqk_fused_qkv_rope_paged_bf16")
+            return out
     B, S, H = x.shape
     D = q_norm_w.shape[0]
     H_Q = w_q.shape[0] // D
@@ -362,6 +381,14 @@ def fused_qkv_rope_ex(
 
     Outputs are shaped ``x.shape[:-1] + (H, D)``.
     """
+    front = _native._front or _native.front()
+    if front is not None:
+        out = front.fused_ex(x, w_q, w_k, w_v, q_norm_w, k_norm_w, cos, sin, positions, cu_seqlens, seq_pos0,
+                             input_norm_w, input_eps, k_cache, v_cache, block_table, kv_seq, kv_pos, return_kv)
+        if out is not None:
+            if type(out) is int:
+                _native.check(out, "mqk_fused_qkv_rope_ex_bf16")
+            return out
     lead, S = _lead_shape(x, cu_seqlens)
     H = x.shape[-1]
     D = q_norm_w.shape[0]

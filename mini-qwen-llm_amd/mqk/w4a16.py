@@ -57,6 +57,13 @@ def w4a16_gemm(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor,
     """``x @ dequant(qweight)``: ``[M, K] bf16 -> [M, N] bf16``."""
     if x.dim() != 2:
         raise ValueError("x must be [M, K]")
+    front = _native._front or _native.front()
+    if front is not None:  # (an ordinary call in C++; None: one for the code below)
+        out = front.gemm(x, qweight, scales, qzeros, group_size)
+        if out is not None:
+            if type(out) is int:
+                _native.check(out, "mqk_w4a16_gemm_ex")
+            return out
     M, K = x.shape
     device = x.device
     x = _require(x, "x", device)
@@ -98,6 +105,8 @@ class LinearW4A16(nn.Module):
         self.register_buffer("qzeros", torch.zeros(G, out_features // 8, dtype=torch.int32))
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        if x.dim() == 2 and x.shape[1] == self.in_features:
+            return w4a16_gemm(x, *_as_int4(self), self.group_size)
         lead = x.shape[:-1]
         out = w4a16_gemm(x.reshape(-1, self.in_features), self.qweight, self.scales, self.qzeros,
                          self.group_size)
@@ -149,6 +158,9 @@ Int4Weights = Tuple[torch.Tensor, torch.Tensor, torch.Tensor]  # (qweight, scale
 
 def _as_int4(p) -> Int4Weights:
     if isinstance(p, LinearW4A16):
+        b = p._buffers  # (where nn.Module's attribute lookup ends up, without its detour)
+        if type(p) is LinearW4A16 and "qweight" in b and "scales" in b and "qzeros" in b:
+            return b["qweight"], b["scales"], b["qzeros"]
         return p.qweight, p.scales, p.qzeros
     qweight, scales, qzeros = p
     return qweight, scales, qzeros
@@ -235,6 +247,24 @@ def fused_qkv_rope_w4a16_ex(
 
 def _fused_w4a16(x, q_proj, k_proj, v_proj, q_norm_w, k_norm_w, cos, sin, positions, group_size,
                  paged=None, return_kv=True, ext_args=None):
+    front = _native._front or _native.front()
+    if front is not None:
+        g = group_size
+        if g is None:
+            g = q_proj.group_size if isinstance(q_proj, LinearW4A16) else 128
+        if ext_args is not None:
+            opt = (ext_args["cu_seqlens"], ext_args["seq_pos0"], ext_args["input_norm_w"], ext_args["input_eps"],
+                   ext_args["k_cache"], ext_args["v_cache"], ext_args["block_table"], ext_args["kv_seq"],
+                   ext_args["kv_pos"])
+        else:
+            opt = (None, None, None, EPS, *(paged or (None,) * 5))
+        out = front.fused_ex_w4(x, *_as_int4(q_proj), *_as_int4(k_proj), *_as_int4(v_proj), q_norm_w, k_norm_w, cos,
+                                sin, positions, *opt, return_kv, g)
+        if out is not None:
+            if type(out) is int:
+                _native.check(out, "mqk_fused_qkv_rope_ex_w4a16" if ext_args is not None else
+                              ("mqk_fused_qkv_rope_w4a16" if paged is None else "mqk_fused_qkv_rope_paged_w4a16"))
+            return out
     lead, S = _lead_shape(x, None if ext_args is None else ext_args.get("cu_seqlens"))
     H = x.shape[-1]
     D = q_norm_w.shape[0]
