@@ -203,6 +203,30 @@ __device__ __forceinline__ T* pick3(int i, T* a, T* b, T* c) {
   return reinterpret_cast<T*>(ua * uintptr_t(i == 0) + ub * uintptr_t(i == 1) + uc * uintptr_t(i == 2));
 }
 
+// pick3 of wave-uniform pointers with the values made opaque instead: the
+// multiplications put ~60 scalar instructions ahead of the decode kernel's first load.
+// (The tile kernels keep pick3: with this form the hidden 1024 T = 1024 call took 17.6-17.8
+// us against 16.5-17.2.)
+template <class T>
+__device__ __forceinline__ T* pick3_uniform(int i, T* a, T* b, T* c) {
+  uintptr_t ua = reinterpret_cast<uintptr_t>(a), ub = reinterpret_cast<uintptr_t>(b),
+            uc = reinterpret_cast<uintptr_t>(c);
+  asm("" : "+s"(ua), "+s"(ub), "+s"(uc));
+  return reinterpret_cast<T*>(i == 0 ? ua : (i == 1 ? ub : uc));
+}
+
+// A load through a pointer that came out of pick3: the arithmetic select hides from the
+// compiler that it is a global address, and it would emit a flat load which the LDS
+// counter waits on too.
+template <class T>
+__device__ __forceinline__ T load_global(const T* ptr) {
+  return *(const __attribute__((address_space(1))) T*)ptr;
+}
+template <class T>
+__device__ __forceinline__ T load_global_nt(const T* ptr) {
+  return __builtin_nontemporal_load((const __attribute__((address_space(1))) T*)ptr);
+}
+
 // Which projection a 128-column tile belongs to: 0 = Q, 1 = K, 2 = V, and the
 // tile's head index inside that projection.
 __device__ __forceinline__ void split_head(int h, int Hq, int Hkv, int& proj, int& hh) {

@@ -34,7 +34,8 @@ constexpr int kDecMaxNK = 16;           // k tiles of one x slice in LDS (64-wid
 // one workgroup per CU with 4 splits of 20 tiles instead of 5 splits over two
 // rounds).
 constexpr int kDecLongMaxNK = 2 * kDecMaxNK;
-constexpr int kDecLookahead = 6;        // weight tiles in flight per wave
+constexpr int kDecLookahead = 6;        // weight tiles in flight per wave (64-row blocks)
+constexpr int kDecLookaheadSmall = 16;  // ... 16- and 32-row blocks, which leave the registers for it
 // Longest k range (in 64-wide tiles) of a split in a launch of several blocks:
 // beyond it the held weights and the finisher no longer fit the 256 VGPRs of a
 // wave without spilling, and such launches run one block each.
@@ -89,8 +90,8 @@ struct XStage {
   __device__ __forceinline__ XStage(const ProblemArgs& p, int64_t kbeg, uint32_t xs_lds, int r0) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    const int part = wave % (2 * MB);
-    first = wave / (2 * MB);
+    const int part = MB == 4 ? wave : wave % (2 * MB);  // (8 waves)
+    first = MB == 4 ? 0 : wave / (2 * MB);
     const int row = part * 8 + (lane >> 3);
     const int gq = (lane & 7) ^ ((row >> 1) & 7);
     const int grow = r0 + row < int(p.M) ? r0 + row : int(p.M) - 1;
@@ -157,7 +158,7 @@ __device__ __forceinline__ float elem_lane(const u32x4_t& v, int i) {
 // Weight fragment load: non-temporal, so the weight stream does not evict the
 // split partials and the x slice from the L2.
 __device__ __forceinline__ u32x4_t wload(const uint16_t* ptr) {
-  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(ptr));
+  return load_global_nt(reinterpret_cast<const u32x4_t*>(ptr));
 }
 
 struct Int4Col {  // this lane's column of an int4 projection
@@ -172,9 +173,9 @@ struct Int4Col {  // this lane's column of an int4 projection
 
 __device__ __forceinline__ Int4Col int4_col(const WeightArgs& w, int proj, int64_t col) {
   const int64_t n = proj == 0 ? w.n_cols[0] : (proj == 1 ? w.n_cols[1] : w.n_cols[2]);
-  return Int4Col{pick3(proj, w.qw[0], w.qw[1], w.qw[2]),
-                 static_cast<const uint16_t*>(pick3(proj, w.sc[0], w.sc[1], w.sc[2])),
-                 pick3(proj, w.qz[0], w.qz[1], w.qz[2]), n, col,
+  return Int4Col{pick3_uniform(proj, w.qw[0], w.qw[1], w.qw[2]),
+                 static_cast<const uint16_t*>(pick3_uniform(proj, w.sc[0], w.sc[1], w.sc[2])),
+                 pick3_uniform(proj, w.qz[0], w.qz[1], w.qz[2]), n, col,
                  w.group, w.scale_fp16 != 0};
 }
 
@@ -205,15 +206,16 @@ __device__ void partial_any(const ProblemArgs& p, const WeightArgs& w, int proj,
     const int64_t k0 = kbeg + int64_t(t) * kBK;
     u32x4_t b[2];
     if constexpr (!INT4) {
-      const uint16_t* wp = pick3(proj, w.w[0], w.w[1], w.w[2]) + col * p.K + k0 + g4 * 8;
-      b[0] = *reinterpret_cast<const u32x4_t*>(wp);
-      b[1] = *reinterpret_cast<const u32x4_t*>(wp + 32);
+      const uint16_t* wp = pick3_uniform(proj, w.w[0], w.w[1], w.w[2]) + col * p.K + k0 + g4 * 8;
+      b[0] = load_global(reinterpret_cast<const u32x4_t*>(wp));
+      b[1] = load_global(reinterpret_cast<const u32x4_t*>(wp + 32));
     } else {
       const Int4Col ic = int4_col(w, proj, col);
       const int64_t grp = k0 / ic.group;
-      const uint32_t q[2] = {uint32_t(ic.qw[(k0 / 8 + g4) * ic.n + col]),
-                             uint32_t(ic.qw[(k0 / 8 + 4 + g4) * ic.n + col])};
-      dequant_tile(ic, q, ic.sc[grp * ic.n + col], uint32_t(ic.qz[grp * (ic.n / 8) + col / 8]), b);
+      const uint32_t q[2] = {uint32_t(load_global(ic.qw + (k0 / 8 + g4) * ic.n + col)),
+                             uint32_t(load_global(ic.qw + (k0 / 8 + 4 + g4) * ic.n + col))};
+      dequant_tile(ic, q, load_global(ic.sc + grp * ic.n + col),
+                   uint32_t(load_global(ic.qz + grp * (ic.n / 8) + col / 8)), b);
     }
     mma_tile<E, MB>(xs, t, b, acc);
   }
@@ -243,15 +245,16 @@ __device__ void partial_any_long(const ProblemArgs& p, const WeightArgs& w, int 
       const int64_t k0 = kbeg + int64_t(t) * kBK;
       u32x4_t b[2];
       if constexpr (!INT4) {
-        const uint16_t* wp = pick3(proj, w.w[0], w.w[1], w.w[2]) + col * p.K + k0 + g4 * 8;
-        b[0] = *reinterpret_cast<const u32x4_t*>(wp);
-        b[1] = *reinterpret_cast<const u32x4_t*>(wp + 32);
+        const uint16_t* wp = pick3_uniform(proj, w.w[0], w.w[1], w.w[2]) + col * p.K + k0 + g4 * 8;
+        b[0] = load_global(reinterpret_cast<const u32x4_t*>(wp));
+        b[1] = load_global(reinterpret_cast<const u32x4_t*>(wp + 32));
       } else {
         const Int4Col ic = int4_col(w, proj, col);
         const int64_t grp = k0 / ic.group;
-        const uint32_t q[2] = {uint32_t(ic.qw[(k0 / 8 + g4) * ic.n + col]),
-                               uint32_t(ic.qw[(k0 / 8 + 4 + g4) * ic.n + col])};
-        dequant_tile(ic, q, ic.sc[grp * ic.n + col], uint32_t(ic.qz[grp * (ic.n / 8) + col / 8]), b);
+        const uint32_t q[2] = {uint32_t(load_global(ic.qw + (k0 / 8 + g4) * ic.n + col)),
+                               uint32_t(load_global(ic.qw + (k0 / 8 + 4 + g4) * ic.n + col))};
+        dequant_tile(ic, q, load_global(ic.sc + grp * ic.n + col),
+                   uint32_t(load_global(ic.qz + grp * (ic.n / 8) + col / 8)), b);
       }
       mma_tile<E, MB>(xs, t, b, acc);
     }
@@ -498,9 +501,10 @@ __device__ __forceinline__ void first_block(const ProblemArgs& p, const WeightAr
   const uint32_t xs_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(xs));
   const int64_t kbeg = int64_t(kt0) * kBK;
   const int64_t col = int64_t(d.hh) * kHeadDim + wave * 16 + c16;
-  constexpr int kLook = NK < kDecLookahead ? NK : kDecLookahead;
+  constexpr int kAhead = MB == 4 ? kDecLookahead : kDecLookaheadSmall;
+  constexpr int kLook = NK < kAhead ? NK : kAhead;
   if constexpr (!INT4) {
-    const uint16_t* wp = pick3(d.proj, w.w[0], w.w[1], w.w[2]) + col * p.K + kbeg + g4 * 8;
+    const uint16_t* wp = pick3_uniform(d.proj, w.w[0], w.w[1], w.w[2]) + col * p.K + kbeg + g4 * 8;
     XStage<MB>(p, kbeg, xs_lds, 0).template all<NK>();
 #pragma unroll
     for (int t = 0; t < kLook; ++t)
@@ -513,6 +517,10 @@ __device__ __forceinline__ void first_block(const ProblemArgs& p, const WeightAr
       if (t + kLook < NK) {
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) hw.b[t + kLook][kk] = wload(wp + (t + kLook) * kBK + kk * 32);
+        // (left free, the compiler sank these loads below the next tiles' MFMAs until
+        // three or four were in flight instead of 2 * kLook: hidden 4096, 32 / 8 heads,
+        // T = 64 19.6 -> 19.0 us in a replayed graph)
+        asm volatile("" ::: "memory");
       }
       mma_tile<E, MB>(xs, t, hw.b[t], acc);
     }
@@ -526,9 +534,9 @@ __device__ __forceinline__ void first_block(const ProblemArgs& p, const WeightAr
       const int64_t k0 = kbeg + int64_t(t) * kBK;
       const int64_t grp = k0 / ic.group;
 #pragma unroll
-      for (int kk = 0; kk < 2; ++kk) q4[t][kk] = uint32_t(ic.qw[(k0 / 8 + kk * 4 + g4) * ic.n + col]);
-      sraw[t] = ic.sc[grp * ic.n + col];
-      zw[t] = uint32_t(ic.qz[grp * (ic.n / 8) + col / 8]);
+      for (int kk = 0; kk < 2; ++kk) q4[t][kk] = uint32_t(load_global(ic.qw + (k0 / 8 + kk * 4 + g4) * ic.n + col));
+      sraw[t] = load_global(ic.sc + grp * ic.n + col);
+      zw[t] = uint32_t(load_global(ic.qz + grp * (ic.n / 8) + col / 8));
     }
     XStage<MB>(p, kbeg, xs_lds, 0).template all<NK>();
     wait_vm<0>();
@@ -668,15 +676,19 @@ __device__ __forceinline__ void run_split_multi(const ProblemArgs& p, const Weig
     }
   };
 
-#pragma unroll 1
-  for (int blk = 0; blk < nblk; ++blk) {
+  // (block 0 ahead of the loop: inside it, what the finish of another iteration may
+  // still have in flight made the compiler wait for every weight load before the first
+  // MFMA: hidden 4096, 32 / 8 heads, T = 128 27.4 -> 25.9 us, T = 300 32.7 -> 32.2)
+  {
     f32x4_t acc[4];
     zero_acc(acc);
-    if (blk == 0) {
-      first_block<Bf16, INT4, 4, NK>(p, w, d, kt0, xs, hw, acc);
-      publish_partial<4>(p, d, 0, acc, part);
-      continue;
-    }
+    first_block<Bf16, INT4, 4, NK>(p, w, d, kt0, xs, hw, acc);
+    publish_partial<4>(p, d, 0, acc, part);
+  }
+#pragma unroll 1
+  for (int blk = 1; blk < nblk; ++blk) {
+    f32x4_t acc[4];
+    zero_acc(acc);
     // this block's x slice in the same LDS once every wave is done with it (the
     // previous block's MFMAs or a finish); the normalising gamma stays in LDS.
     // Once its first tiles have landed, so have the previous block's partial
@@ -761,8 +773,8 @@ __device__ __forceinline__ DecWork dec_work(const ProblemArgs& p, const Epilogue
   d.nblk = int((p.M + ROWS - 1) / ROWS);
   split_head(d.head, e.Hq, e.Hkv, d.proj, d.hh);
   d.H = d.proj == 0 ? e.Hq : e.Hkv;
-  d.gamma = pick3(d.proj, e.q_gamma, e.k_gamma, e.k_gamma);
-  d.out = pick3(d.proj, e.q, e.k, e.v);
+  d.gamma = pick3_uniform(d.proj, e.q_gamma, e.k_gamma, e.k_gamma);
+  d.out = pick3_uniform(d.proj, e.q, e.k, e.v);
   // (XCC_ID is the physical XCD; a partition of the GPU holds xcds of them)
   d.inc = arrival_inc(xcc_id() % xcds, (ctl & 1) != 0);
   d.max_spins = ctl >> 1;
@@ -795,12 +807,12 @@ __device__ __forceinline__ void decode_body(const ProblemArgs& p, const WeightAr
   block_rows<MB>(e, d, int(p.M), 0, prow, cslot);
   f32x4_t acc[MB];
   zero_acc<MB>(acc);
-  auto stream = [&](auto n) __attribute__((always_inline)) {
-    HeldWeights<decltype(n)::value> hw;
-    first_block<E, INT4, MB, decltype(n)::value>(p, w, d, kt0, xs, hw, acc);
-  };
-#define MQK_DEC_CASE(n) \
-  case n: stream(std::integral_constant<int, n>{}); break;
+#define MQK_DEC_CASE(n)                                       \
+  case n: {                                                   \
+    HeldWeights<n> hw;                                        \
+    first_block<E, INT4, MB, n>(p, w, d, kt0, xs, hw, acc);   \
+    break;                                                    \
+  }
 #define MQK_DEC_CASES_16                                              \
   MQK_DEC_CASE(1) MQK_DEC_CASE(2) MQK_DEC_CASE(3) MQK_DEC_CASE(4)     \
   MQK_DEC_CASE(5) MQK_DEC_CASE(6) MQK_DEC_CASE(7) MQK_DEC_CASE(8)     \
@@ -847,13 +859,13 @@ __device__ __forceinline__ void decode_long_body(const ProblemArgs& p, const Wei
   block_rows<MB>(e, d, int(p.M), 0, prow, cslot);
   f32x4_t acc[MB];
   zero_acc<MB>(acc);
-  auto slice = [&](auto n, int from) __attribute__((always_inline)) {
-    HeldWeights<decltype(n)::value> hw;
-    first_block<E, INT4, MB, decltype(n)::value>(p, w, d, kt0 + from, xs, hw, acc);
-  };
   const int n1 = INT4 ? (nk + 1) / 2 : kDecMaxNK;
-#define MQK_DEC_SLICE(n) \
-  case n: slice(std::integral_constant<int, n>{}, from); break;
+#define MQK_DEC_SLICE(n)                                             \
+  case n: {                                                          \
+    HeldWeights<n> hw;                                               \
+    first_block<E, INT4, MB, n>(p, w, d, kt0 + from, xs, hw, acc);   \
+    break;                                                           \
+  }
 #define MQK_DEC_SLICES_8_16                                                              \
   MQK_DEC_SLICE(8) MQK_DEC_SLICE(9) MQK_DEC_SLICE(10) MQK_DEC_SLICE(11) MQK_DEC_SLICE(12) \
   MQK_DEC_SLICE(13) MQK_DEC_SLICE(14) MQK_DEC_SLICE(15) MQK_DEC_SLICE(16)
@@ -868,7 +880,10 @@ __device__ __forceinline__ void decode_long_body(const ProblemArgs& p, const Wei
       }
     }
   } else {
-    slice(std::integral_constant<int, kDecMaxNK>{}, 0);
+    {
+      HeldWeights<kDecMaxNK> hw;
+      first_block<E, INT4, MB, kDecMaxNK>(p, w, d, kt0, xs, hw, acc);
+    }
     __syncthreads();
     const int from = n1;
     switch (nk - n1) {

@@ -42,9 +42,9 @@ w4_unpack_kernel(WeightArgs w, int64_t K, uint16_t* __restrict__ out) {
     }
   }
   const int64_t N = proj == 0 ? w.n_cols[0] : (proj == 1 ? w.n_cols[1] : w.n_cols[2]);
-  const int32_t* qw = pick3<const int32_t>(proj, w.qw[0], w.qw[1], w.qw[2]);
-  const int32_t* qz = pick3<const int32_t>(proj, w.qz[0], w.qz[1], w.qz[2]);
-  const uint16_t* sc = pick3<const uint16_t>(proj, static_cast<const uint16_t*>(w.sc[0]),
+  const int32_t* qw = pick3_uniform<const int32_t>(proj, w.qw[0], w.qw[1], w.qw[2]);
+  const int32_t* qz = pick3_uniform<const int32_t>(proj, w.qz[0], w.qz[1], w.qz[2]);
+  const uint16_t* sc = pick3_uniform<const uint16_t>(proj, static_cast<const uint16_t*>(w.sc[0]),
                                              static_cast<const uint16_t*>(w.sc[1]), static_cast<const uint16_t*>(w.sc[2]));
   const int64_t j0 = int64_t(blockIdx.y) * kWords;
   const int nj = int(K / 8 - j0 < kWords ? K / 8 - j0 : kWords);
@@ -54,14 +54,14 @@ w4_unpack_kernel(WeightArgs w, int64_t K, uint16_t* __restrict__ out) {
 #pragma unroll
   for (int i = 0; i < kWords / 4; ++i) {
     const int j = wave + 4 * i;
-    r[i] = j < nj ? uint32_t(qw[(j0 + j) * N + c0 + lane]) : 0u;
+    r[i] = j < nj ? uint32_t(load_global(qw + (j0 + j) * N + c0 + lane)) : 0u;
   }
 #pragma unroll
   for (int i = 0; i < kWords / 4; ++i) words[wave + 4 * i][lane] = r[i];
   for (int g = wave; g < ng; g += 4) {
     const int64_t col = c0 + lane;
-    const uint32_t sraw = sc[(g0 + g) * N + col];
-    const uint32_t zw = uint32_t(qz[(g0 + g) * (N / 8) + col / 8]);
+    const uint32_t sraw = load_global(sc + (g0 + g) * N + col);
+    const uint32_t zw = uint32_t(load_global(qz + (g0 + g) * (N / 8) + col / 8));
     scale[g][lane] = w.scale_fp16 ? f16_to_f32(sraw) : bf16_to_f32(sraw);
     zero[g][lane] = float((zw >> ((col % 8) * 4)) & 0xFu);
   }
