@@ -963,10 +963,8 @@ static int fused_f32_impl(bool half, const void* x, const void* w_q, const void*
   a.q = q;
   a.k = k;
   a.v = v;
-  // 16-row tiles when 32-row tiles would leave CUs idle
   const Topology topo = device_topology();
-  const int rows = (T + 31) / 32 * (Hq + 2 * Hkv) < topo.cus ? 16 : 32;
-  return hip_status(launch_f32_qkv(a, rows, half, topo.xcds, static_cast<hipStream_t>(stream)),
+  return hip_status(launch_f32_qkv(a, half, topo.cus, topo.xcds, static_cast<hipStream_t>(stream)),
                     half ? "f16 front launch" : "f32 front launch");
 }
 

@@ -252,7 +252,7 @@ struct F32Args {
   int head_dim = kHeadDimDefault;
 };
 constexpr int kF32BK = 32;       // k extent of one staged tile of the fp32 / fp16 front
-// rows: token rows per workgroup, 32 or 16; half: fp16 elements (else fp32)
-hipError_t launch_f32_qkv(const F32Args& a, int rows, bool half, int xcds, hipStream_t stream);
+// half: fp16 elements (else fp32)
+hipError_t launch_f32_qkv(const F32Args& a, bool half, int cus, int xcds, hipStream_t stream);
 
 }  // namespace mqk
