@@ -249,12 +249,15 @@ __device__ __forceinline__ int xcd_tile_id(int bid, int nblocks, int xcds) {
 
 // L2 -> LDS: this lane's 16 bytes at gptr go to LDS byte lds_base + 16 * lane
 // (lds_base wave-uniform).  M0 carries the LDS base; it is saved and restored
-// around the load because the compiler reserves it.
+// around the load because the compiler reserves it.  The s_nop is required: a scalar
+// write of M0 needs one wait state before a load to the LDS, and the compiler inserts
+// none inside asm.
 __device__ __forceinline__ void dma16(const void* gptr, uint32_t lds_base) {
   uint32_t saved;
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dwordx4 %2, off\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(saved)
@@ -269,6 +272,7 @@ __device__ __forceinline__ void dma4(const void* gptr, uint32_t lds_base) {
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dword %2, off\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(saved)
@@ -288,6 +292,7 @@ __device__ __forceinline__ void dma16_at(const void* gptr, uint32_t lds_base) {
   asm volatile(
       "s_mov_b32 %0, m0\n\t"
       "s_mov_b32 m0, %1\n\t"
+      "s_nop 0\n\t"
       "global_load_lds_dwordx4 %2, off offset:%3\n\t"
       "s_mov_b32 m0, %0"
       : "=&s"(saved)
