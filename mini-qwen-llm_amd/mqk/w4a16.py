@@ -248,7 +248,8 @@ def fused_qkv_rope_w4a16_ex(
 def _fused_w4a16(x, q_proj, k_proj, v_proj, q_norm_w, k_norm_w, cos, sin, positions, group_size,
                  paged=None, return_kv=True, ext_args=None):
     front = _native._front or _native.front()
-    if front is not None:
+    # (a paged call without its cache is refused below; to the extension no cache is the _ex form without one)
+    if front is not None and (paged is None or paged[0] is not None):
         g = group_size
         if g is None:
             g = q_proj.group_size if isinstance(q_proj, LinearW4A16) else 128

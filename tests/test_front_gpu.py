@@ -142,6 +142,11 @@ def test_ex_and_paged_forms(device):
             _same(lambda: paged(positions=pos, kv_seq=seq, kv_pos=at, return_kv=kv), f"paged positions D={D} {kv}")
             _same(lambda: ex(cache=True, input_norm_w=gin, positions=pos, kv_seq=seq, kv_pos=at, return_kv=kv), f"ex D={D}")
         _same(lambda: paged(positions=pos), "positions without slots")
+        none = {"k_cache": None, "v_cache": None, "block_table": None}
+        for kw in (none, {**none, "return_kv": False}, {**none, "positions": pos, "kv_seq": seq, "kv_pos": at},
+                   {**_paged(device, D), "k_cache": None}, {**_paged(device, D), "block_table": None}):
+            _same(lambda: mqk.fused_qkv_rope_paged(**b, **kw), "paged without a cache")
+            assert isinstance(_outcome(lambda: mqk.fused_qkv_rope_paged(**b, **kw))[0], type), "refused"
         _same(lambda: paged(positions=pos, kv_seq=seq.long(), kv_pos=at.long()), "int64 slots")
         _same(ex, "plain ex")
         _same(lambda: ex(return_kv=False), "no cache, no kv")
@@ -196,6 +201,11 @@ def test_w4a16_forms(device):
             out = mqk.fused_qkv_rope_w4a16_paged(b["x"], *mods, *rope, **p)
             return (*out, p["k_cache"], p["v_cache"])
         _same(paged, f"paged D={D}")
+        for p in (dict.fromkeys(_paged(device, D)), {**_paged(device, D), "v_cache": None},
+                  {**dict.fromkeys(_paged(device, D)), "return_kv": False}):
+            call = lambda: mqk.fused_qkv_rope_w4a16_paged(b["x"], *mods, *rope, **p)
+            _same(call, "paged without a cache")
+            assert isinstance(_outcome(call)[0], type), "refused"
         _same(lambda: mqk.fused_qkv_rope_w4a16(b["x"], *w, *rope, group_size=64), "wrong group")
         _same(lambda: mqk.fused_qkv_rope_w4a16(b["x"], *w, *rope, group_size=0), "group 0")
         _same(lambda: mqk.fused_qkv_rope_w4a16(b["x"], *w, *rope, group_size=True), "boolean group")
