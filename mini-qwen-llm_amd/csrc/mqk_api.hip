@@ -379,6 +379,17 @@ size_t unpack_bytes(int64_t M, int64_t K, int n_tiles) {
   return g_prefill_tile.load() == 0 ? n : 0;  // (a requested int4 tile variant is run)
 }
 
+// Held from the launch that writes normalised rows, their scales or unpacked weights to
+// a workspace until the launch that reads them: two threads may call on one stream, and
+// so with one workspace (the mqk package's is the stream's), and without it the second
+// thread's first launch could come between the first's two.  (Recursive: a call can hold
+// it for its weights and for its rows.  Workspaces share 64 locks.)
+std::recursive_mutex g_handover[64];
+std::unique_lock<std::recursive_mutex> handover_lock(const void* workspace) {
+  const uintptr_t a = reinterpret_cast<uintptr_t>(workspace) >> 9;
+  return std::unique_lock<std::recursive_mutex>(g_handover[(a ^ (a >> 6) ^ (a >> 12)) % 64]);
+}
+
 // Common launcher of the fused op (bf16 or int4 weights).  With an input norm
 // (p.in_gamma set, epsilon in_eps), a pre-pass first writes the normalised rows to
 // the workspace after the plan's region, and the plan runs on them; a workspace
@@ -396,6 +407,7 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     const size_t rows = p.in_gamma ? std::max(norm_ahead_bytes(p.M, p.K), align_up(size_t(p.M) * sizeof(float), 256)) : 0;
     if (epilogue_aligned(e) && off >= align_up(plan_region(pl, p.M, p.n_tiles), 256) + rows) {
       uint16_t* wt = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
+      const auto lock = handover_lock(workspace);
       const int st = hip_status(launch_w4_unpack(w, p.n_tiles, p.K, wt, stream), "int4 weight unpack launch");
       if (st != MQK_OK) return st;
       WeightArgs wu{};
@@ -415,6 +427,7 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     const size_t off = align_up(plan_region(pl, p.M, p.n_tiles), 256);
     if (ws_bytes >= off + norm_ahead_bytes(p.M, p.K)) {
       uint16_t* xn = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
+      const auto lock = handover_lock(workspace);
       const int st = hip_status(launch_row_scale(p.x, p.in_gamma, p.M, p.K, in_eps, nullptr, xn, stream),
                                 "input norm pre-pass launch");
       if (st != MQK_OK) return st;
@@ -472,7 +485,9 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
   if (need > 0 && (!workspace || ws_bytes < need))
     return fail(MQK_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given%s", need, ws_bytes,
                 workspace ? "" : " (NULL)");
+  std::unique_lock<std::recursive_mutex> lock;
   if (p.in_gamma) {
+    lock = handover_lock(workspace);
     float* scale = reinterpret_cast<float*>(static_cast<char*>(workspace) + scale_off);
     const int st = hip_status(launch_row_scale(p.x, p.in_gamma, p.M, p.K, in_eps, scale, nullptr, stream),
                               "input norm pre-pass launch");
@@ -796,6 +811,7 @@ static int fused_bf16_any_d(const mqk_bf16* x, const mqk_bf16* w_q, const mqk_bf
     }
   }
   ProblemArgs pn{x, T, hidden, 0};
+  std::unique_lock<std::recursive_mutex> lock;
   if (ext && ext->in_gamma) {
     if ((st = apply_ext(ext, positions, S, T, pn, er)) != MQK_OK) return st;  // (in_gamma checks)
     // the scales after the workspace's arrival counters, which other calls on it need at zero
@@ -803,6 +819,7 @@ static int fused_bf16_any_d(const mqk_bf16* x, const mqk_bf16* w_q, const mqk_bf
     if (!workspace || ws_bytes < off + size_t(T) * sizeof(float))
       return fail(MQK_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given%s", off + size_t(T) * sizeof(float),
                   ws_bytes, workspace ? "" : " (NULL)");
+    lock = handover_lock(workspace);
     float* scale = reinterpret_cast<float*>(static_cast<char*>(workspace) + off);
     st = hip_status(launch_row_scale(x, nullptr, T, hidden, ext->in_eps, scale, nullptr, hs), "input norm pre-pass launch");
     if (st != MQK_OK) return st;
