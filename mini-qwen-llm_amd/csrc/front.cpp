@@ -15,6 +15,10 @@
 // tensor to copy or convert, another device, a workspace to make -- returns None, and
 // the Python code beside it, which remains the definition of the entry point, takes
 // the call.  A native failure returns the status for Python to raise.
+//
+// The GIL is released where a call can wait for the driver: the output allocations and
+// the launches (a full queue, or one whose host function needs the GIL).  Every pointer
+// is read from its tensor before; 0.1 us of a call.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -90,6 +94,23 @@ struct Call {
   }
 };
 
+// Without the GIL while it lives.  Nothing in its scope touches a Python object.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  ~Unlocked() { PyEval_RestoreThread(state_); }
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+
+template <class T>
+const T* ptr(const at::Tensor* t) {
+  return static_cast<const T*>(t->data_ptr());
+}
+
 bool current_device_is(c10::DeviceIndex dev) {
   static const c10::impl::VirtualGuardImpl guard(c10::DeviceType::CUDA);
   return guard.getDevice().index() == dev;
@@ -110,9 +131,12 @@ PyObject* stream_of(c10::DeviceIndex dev) {
 
 // The workspace of (dev, stream) if it holds n bytes; none needed for n == 0.  False:
 // absent or too small (Python makes or grows it).
-bool workspace(c10::DeviceIndex dev, PyObject* stream, size_t n, void** ptr, size_t* bytes) {
-  *ptr = nullptr;
-  *bytes = 0;
+struct Workspace {
+  at::Tensor buf;  // (held: another thread may replace it while the GIL is released)
+  void* ptr = nullptr;
+  size_t bytes = 0;
+};
+bool workspace(c10::DeviceIndex dev, PyObject* stream, size_t n, Workspace* ws) {
   if (n == 0) return true;
   PyObject* key = Py_BuildValue("(iO)", int(dev), stream);
   if (!key) {
@@ -124,8 +148,9 @@ bool workspace(c10::DeviceIndex dev, PyObject* stream, size_t n, void** ptr, siz
   if (!buf || !THPVariable_Check(buf)) return false;
   const at::Tensor& t = THPVariable_Unpack(buf);
   if (size_t(t.numel()) < n) return false;
-  *ptr = t.data_ptr();
-  *bytes = size_t(t.numel());
+  ws->buf = t;
+  ws->ptr = t.data_ptr();
+  ws->bytes = size_t(t.numel());
   return true;
 }
 
@@ -210,26 +235,32 @@ PyObject* fused(PyObject*, PyObject* const* a, Py_ssize_t n) {
   size_t need = 0;
   if (type == at::kBFloat16) need = g_lib.size(T, bq, bkv, H);
   else if (type == at::kHalf) need = g_lib.f16_size(T, int(hq), int(hkv), H, int(D));
-  void* ws;
-  size_t ws_bytes;
-  const bool have = workspace(c.dev, stream, need, &ws, &ws_bytes);
+  Workspace ws;
+  const bool have = workspace(c.dev, stream, need, &ws);
   void* hs = PyLong_AsVoidPtr(stream);
   Py_DECREF(stream);
   if (!have) return none();
-  at::Tensor q = fresh({B, S, hq, D}, type, c.dev), k = fresh({B, S, hkv, D}, type, c.dev),
-             v = fresh({B, S, hkv, D}, type, c.dev);
+  const void* in[8] = {x->data_ptr(),    w[0]->data_ptr(), w[1]->data_ptr(),  w[2]->data_ptr(),
+                       r.gq->data_ptr(), r.gk->data_ptr(), r.cos->data_ptr(), r.sin->data_ptr()};
+  at::Tensor q, k, v;
   int st;
-  if (type == at::kFloat) {
-    auto p = [](const at::Tensor* t) { return static_cast<const float*>(t->data_ptr()); };
-    st = g_lib.f32(p(x), p(w[0]), p(w[1]), p(w[2]), p(r.gq), p(r.gk), p(r.cos), p(r.sin), pos, T, S, H, int(hq), int(hkv),
-                   int(D), r.rows, kEps, static_cast<float*>(q.data_ptr()), static_cast<float*>(k.data_ptr()),
-                   static_cast<float*>(v.data_ptr()), hs);
-  } else {
-    auto p = [](const at::Tensor* t) { return static_cast<const uint16_t*>(t->data_ptr()); };
-    auto o = [](at::Tensor& t) { return static_cast<uint16_t*>(t.data_ptr()); };
-    const auto fn = type == at::kHalf ? g_lib.f16 : g_lib.bf16;
-    st = fn(p(x), p(w[0]), p(w[1]), p(w[2]), p(r.gq), p(r.gk), p(r.cos), p(r.sin), pos, T, S, H, int(hq), int(hkv), int(D),
-            r.rows, kEps, o(q), o(k), o(v), ws, ws_bytes, hs);
+  {
+    Unlocked unlocked;
+    q = fresh({B, S, hq, D}, type, c.dev);
+    k = fresh({B, S, hkv, D}, type, c.dev);
+    v = fresh({B, S, hkv, D}, type, c.dev);
+    if (type == at::kFloat) {
+      auto p = [&](int i) { return static_cast<const float*>(in[i]); };
+      st = g_lib.f32(p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), pos, T, S, H, int(hq), int(hkv), int(D), r.rows, kEps,
+                     static_cast<float*>(q.data_ptr()), static_cast<float*>(k.data_ptr()),
+                     static_cast<float*>(v.data_ptr()), hs);
+    } else {
+      auto p = [&](int i) { return static_cast<const uint16_t*>(in[i]); };
+      auto o = [](at::Tensor& t) { return static_cast<uint16_t*>(t.data_ptr()); };
+      const auto fn = type == at::kHalf ? g_lib.f16 : g_lib.bf16;
+      st = fn(p(0), p(1), p(2), p(3), p(4), p(5), p(6), p(7), pos, T, S, H, int(hq), int(hkv), int(D), r.rows, kEps, o(q),
+              o(k), o(v), ws.ptr, ws.bytes, hs);
+    }
   }
   if (st != 0) return PyLong_FromLong(st);
   return wrap3(std::move(q), std::move(k), std::move(v));
@@ -309,17 +340,17 @@ bool lead_shape(const at::Tensor& x, bool varlen, int64_t* lead, int* n_lead, in
 // Outputs [*lead, heads, D] in bf16 (k and v undefined without return_kv).
 struct Outputs {
   at::Tensor q, k, v;
-  Outputs(const int64_t* lead, int n_lead, int64_t hq, int64_t hkv, int64_t D, bool kv, c10::DeviceIndex dev) {
+  void make(const int64_t* lead, int n_lead, int64_t hq, int64_t hkv, int64_t D, bool kv, c10::DeviceIndex dev) {
     int64_t s[4] = {lead[0], lead[1], 0, 0};
-    auto make = [&](int64_t h) {
+    auto one = [&](int64_t h) {
       s[n_lead] = h;
       s[n_lead + 1] = D;
       return fresh(at::IntArrayRef(s, size_t(n_lead) + 2), at::kBFloat16, dev);
     };
-    q = make(hq);
+    q = one(hq);
     if (kv) {
-      k = make(hkv);
-      v = make(hkv);
+      k = one(hkv);
+      v = one(hkv);
     }
   }
   static uint16_t* ptr(const at::Tensor& t) { return t.defined() ? static_cast<uint16_t*>(t.data_ptr()) : nullptr; }
@@ -349,16 +380,21 @@ PyObject* fused_ex(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!e.read(c, a + 8, T, H, hkv, D) || !current_device_is(c.dev)) return none();
   PyObject* stream = stream_of(c.dev);
   if (!stream) return nullptr;
-  void* ws;
-  size_t ws_bytes;
-  const bool have = workspace(c.dev, stream, g_lib.ex_size(T, bq, bkv, H, &e.ext), &ws, &ws_bytes);
+  Workspace ws;
+  const bool have = workspace(c.dev, stream, g_lib.ex_size(T, bq, bkv, H, &e.ext), &ws);
   void* hs = PyLong_AsVoidPtr(stream);
   Py_DECREF(stream);
   if (!have) return none();
-  Outputs o(lead, n_lead, hq, hkv, D, e.return_kv, c.dev);
-  auto p = [](const at::Tensor* t) { return static_cast<const uint16_t*>(t->data_ptr()); };
-  const int st = g_lib.ex(p(x), p(w[0]), p(w[1]), p(w[2]), p(r.gq), p(r.gk), p(r.cos), p(r.sin), e.pos, T, S, H, int(hq),
-                          int(hkv), int(D), r.rows, kEps, o.ptr(o.q), o.ptr(o.k), o.ptr(o.v), &e.ext, ws, ws_bytes, hs);
+  const uint16_t* in[8] = {ptr<uint16_t>(x),    ptr<uint16_t>(w[0]), ptr<uint16_t>(w[1]),  ptr<uint16_t>(w[2]),
+                           ptr<uint16_t>(r.gq), ptr<uint16_t>(r.gk), ptr<uint16_t>(r.cos), ptr<uint16_t>(r.sin)};
+  Outputs o;
+  int st;
+  {
+    Unlocked unlocked;
+    o.make(lead, n_lead, hq, hkv, D, e.return_kv, c.dev);
+    st = g_lib.ex(in[0], in[1], in[2], in[3], in[4], in[5], in[6], in[7], e.pos, T, S, H, int(hq), int(hkv), int(D), r.rows,
+                  kEps, o.ptr(o.q), o.ptr(o.k), o.ptr(o.v), &e.ext, ws.ptr, ws.bytes, hs);
+  }
   if (st != 0) return PyLong_FromLong(st);
   return wrap3(std::move(o.q), std::move(o.k), std::move(o.v));
   END_HANDLE_TH_ERRORS
@@ -415,19 +451,29 @@ PyObject* fused_ex_w4(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (!e.read(c, a + 14, T, H, hkv, D) || !current_device_is(c.dev)) return none();
   PyObject* stream = stream_of(c.dev);
   if (!stream) return nullptr;
-  void* ws;
-  size_t ws_bytes;
-  const bool have = workspace(c.dev, stream, g_lib.w4_size(T, bq, bkv, H, &e.ext), &ws, &ws_bytes);
+  Workspace ws;
+  const bool have = workspace(c.dev, stream, g_lib.w4_size(T, bq, bkv, H, &e.ext), &ws);
   void* hs = PyLong_AsVoidPtr(stream);
   Py_DECREF(stream);
   if (!have) return none();
-  Outputs o(lead, n_lead, hq, hkv, D, e.return_kv, c.dev);
-  auto p = [](const at::Tensor* t) { return static_cast<const uint16_t*>(t->data_ptr()); };
-  auto i32 = [](const at::Tensor* t) { return t->data_ptr<int32_t>(); };
-  const int st = g_lib.ex_w4(p(x), i32(w[0].qw), w[0].sc->data_ptr(), i32(w[0].qz), i32(w[1].qw), w[1].sc->data_ptr(),
-                             i32(w[1].qz), i32(w[2].qw), w[2].sc->data_ptr(), i32(w[2].qz), int(g), w[0].scale_type, p(r.gq),
-                             p(r.gk), p(r.cos), p(r.sin), e.pos, T, S, H, int(hq), int(hkv), int(D), r.rows, kEps, o.ptr(o.q),
-                             o.ptr(o.k), o.ptr(o.v), &e.ext, ws, ws_bytes, hs);
+  const uint16_t* in[5] = {ptr<uint16_t>(x), ptr<uint16_t>(r.gq), ptr<uint16_t>(r.gk), ptr<uint16_t>(r.cos),
+                           ptr<uint16_t>(r.sin)};
+  const int32_t *qw[3], *qz[3];
+  const void* sc[3];
+  for (int i = 0; i < 3; ++i) {
+    qw[i] = ptr<int32_t>(w[i].qw);
+    sc[i] = w[i].sc->data_ptr();
+    qz[i] = ptr<int32_t>(w[i].qz);
+  }
+  Outputs o;
+  int st;
+  {
+    Unlocked unlocked;
+    o.make(lead, n_lead, hq, hkv, D, e.return_kv, c.dev);
+    st = g_lib.ex_w4(in[0], qw[0], sc[0], qz[0], qw[1], sc[1], qz[1], qw[2], sc[2], qz[2], int(g), w[0].scale_type, in[1],
+                     in[2], in[3], in[4], e.pos, T, S, H, int(hq), int(hkv), int(D), r.rows, kEps, o.ptr(o.q), o.ptr(o.k),
+                     o.ptr(o.v), &e.ext, ws.ptr, ws.bytes, hs);
+  }
   if (st != 0) return PyLong_FromLong(st);
   return wrap3(std::move(o.q), std::move(o.k), std::move(o.v));
   END_HANDLE_TH_ERRORS
@@ -446,16 +492,22 @@ PyObject* gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   if (M == 0 || !group_of(a[4], K, &g) || !w.read(c, a + 1, K, g) || !current_device_is(c.dev)) return none();
   PyObject* stream = stream_of(c.dev);
   if (!stream) return nullptr;
-  void* ws;
-  size_t ws_bytes;
-  const bool have = workspace(c.dev, stream, g_lib.gemm_size(M, K, w.N), &ws, &ws_bytes);
+  Workspace ws;
+  const bool have = workspace(c.dev, stream, g_lib.gemm_size(M, K, w.N), &ws);
   void* hs = PyLong_AsVoidPtr(stream);
   Py_DECREF(stream);
   if (!have) return none();
-  at::Tensor out = fresh({M, w.N}, at::kBFloat16, c.dev);
-  const int st = g_lib.gemm(static_cast<const uint16_t*>(x->data_ptr()), w.qw->data_ptr<int32_t>(), w.sc->data_ptr(),
-                            w.qz->data_ptr<int32_t>(), M, K, w.N, int(g), w.scale_type,
-                            static_cast<uint16_t*>(out.data_ptr()), ws, ws_bytes, hs);
+  const uint16_t* xp = ptr<uint16_t>(x);
+  const int32_t *qw = ptr<int32_t>(w.qw), *qz = ptr<int32_t>(w.qz);
+  const void* sc = w.sc->data_ptr();
+  at::Tensor out;
+  int st;
+  {
+    Unlocked unlocked;
+    out = fresh({M, w.N}, at::kBFloat16, c.dev);
+    st = g_lib.gemm(xp, qw, sc, qz, M, K, w.N, int(g), w.scale_type, static_cast<uint16_t*>(out.data_ptr()), ws.ptr,
+                    ws.bytes, hs);
+  }
   if (st != 0) return PyLong_FromLong(st);
   return THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS

@@ -77,3 +77,52 @@ def test_threads_on_one_stream(make, calls, front, device, monkeypatch):
     for t in threads:
         t.join()
     assert wrong.tolist() == [0, 0], "calls with another thread's rows or weights"
+
+
+def test_the_front_lets_other_threads_run(device):
+    """The C++ front releases the GIL around its allocations and launches: with a switch
+    interval that no thread outwaits, another Python thread gets on only while a call
+    waits for the driver."""
+    import sys
+    from mqk import _native
+    import mqk
+    ext = _native.front()
+    hidden, Hq, Hkv, T = 256, 2, 1, 4
+    w = [torch.zeros(h * D, hidden, dtype=torch.bfloat16, device=device) for h in (Hq, Hkv, Hkv)]
+    x = torch.zeros(1, T, hidden, dtype=torch.bfloat16, device=device)
+    gam = torch.ones(hidden, dtype=torch.bfloat16, device=device)
+    int4 = [(torch.zeros(hidden // 8, h * D, dtype=torch.int32, device=device),
+             torch.ones(2, h * D, dtype=torch.float16, device=device),
+             torch.zeros(2, h * D // 8, dtype=torch.int32, device=device)) for h in (Hq, Hkv, Hkv)]
+    rope = _rope(T, device)
+    opt = (None, None, None, gam, 1e-6) + (None,) * 5 + (True,)
+    calls = {"fused": (x, *w, *rope, None), "fused_ex": (x, *w, *rope, *opt),
+             "fused_ex_w4": (x, *(t for p in int4 for t in p), *rope, *opt, 128),
+             "gemm": (x[0], *int4[0], 128)}
+    mqk.fused_qkv_rope_ex(x, *w, *rope, input_norm_w=gam)  # (the workspace)
+    mqk.w4a16_gemm(x[0], *int4[0])
+    old = sys.getswitchinterval()
+    for name, args in calls.items():
+        fn, seen, stop = getattr(ext, name), [0], []
+        assert type(fn(*args)) in (tuple, torch.Tensor), name
+        torch.cuda.synchronize()
+
+        def count():
+            while not stop:
+                seen[0] += 1
+                _native.version()  # (ctypes: gives the GIL up, and must get it again)
+        sys.setswitchinterval(1000.0)
+        try:
+            t = threading.Thread(target=count)
+            t.start()
+            before = seen[0]
+            keep = []
+            while seen[0] < before + 20 and len(keep) < 3000:
+                keep.append(fn(*args))
+            got = seen[0] - before
+        finally:
+            stop.append(1)
+            sys.setswitchinterval(old)
+            t.join()
+        assert got >= 20, f"{name}: {got} turns of the other thread in {len(keep)} calls"
+        torch.cuda.synchronize()
