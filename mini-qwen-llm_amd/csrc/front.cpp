@@ -51,6 +51,7 @@ struct Lib {
 PyObject* g_workspaces = nullptr;  // mqk._native._workspaces: {(device index, stream): uint8 tensor}
 PyObject* g_raw_stream = nullptr;  // torch's raw current-stream accessor
 PyObject* g_parameter = nullptr;   // torch.nn.Parameter
+PyObject* g_capturing = nullptr;   // mqk._native.capturing: is the current stream being captured?
 bool g_bound = false;
 
 constexpr float kEps = 1e-6f;  // the op's fixed QK-Norm epsilon
@@ -154,6 +155,18 @@ bool workspace(c10::DeviceIndex dev, PyObject* stream, size_t n, Workspace* ws) 
   return true;
 }
 
+// Whether the current stream is being captured (also when that cannot be told).
+bool capturing() {
+  PyObject* r = PyObject_CallNoArgs(g_capturing);
+  if (!r) {
+    PyErr_Clear();
+    return true;
+  }
+  const bool yes = r != Py_False;
+  Py_DECREF(r);
+  return yes;
+}
+
 // head_dim 64 and 128 (128-column blocks of whole heads) are taken here; other sizes in Python.
 bool blocks_of(int64_t D, int64_t hq, int64_t hkv, int* bq, int* bkv) {
   if (D != 128 && D != 64) return false;
@@ -235,6 +248,10 @@ PyObject* fused(PyObject*, PyObject* const* a, Py_ssize_t n) {
   size_t need = 0;
   if (type == at::kBFloat16) need = g_lib.size(T, bq, bkv, H);
   else if (type == at::kHalf) need = g_lib.f16_size(T, int(hq), int(hkv), H, int(D));
+  if (type == at::kHalf && need > 0 && capturing()) {  // (a workspace of the graph's own: Python)
+    Py_DECREF(stream);
+    return none();
+  }
   Workspace ws;
   const bool have = workspace(c.dev, stream, need, &ws);
   void* hs = PyLong_AsVoidPtr(stream);
@@ -452,7 +469,10 @@ PyObject* fused_ex_w4(PyObject*, PyObject* const* a, Py_ssize_t n) {
   PyObject* stream = stream_of(c.dev);
   if (!stream) return nullptr;
   Workspace ws;
-  const bool have = workspace(c.dev, stream, g_lib.w4_size(T, bq, bkv, H, &e.ext), &ws);
+  const size_t need = g_lib.w4_size(T, bq, bkv, H, &e.ext);
+  // (a captured call that unpacks its weights has a workspace of the graph's own: Python)
+  const bool own = need > g_lib.ex_size(T, bq, bkv, H, &e.ext) && capturing();
+  const bool have = !own && workspace(c.dev, stream, need, &ws);
   void* hs = PyLong_AsVoidPtr(stream);
   Py_DECREF(stream);
   if (!have) return none();
@@ -513,10 +533,11 @@ PyObject* gemm(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
-// bind(dlopen handle of libmqk.so, workspaces dict, raw-stream accessor, Parameter class)
+// bind(dlopen handle of libmqk.so, workspaces dict, raw-stream accessor, Parameter class,
+// capture check)
 PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
-  if (n != 4 || !PyDict_Check(a[1]) || !PyCallable_Check(a[2]) || !PyType_Check(a[3])) {
-    PyErr_SetString(PyExc_TypeError, "bind(handle, workspaces, raw_stream, parameter_class)");
+  if (n != 5 || !PyDict_Check(a[1]) || !PyCallable_Check(a[2]) || !PyType_Check(a[3]) || !PyCallable_Check(a[4])) {
+    PyErr_SetString(PyExc_TypeError, "bind(handle, workspaces, raw_stream, parameter_class, capturing)");
     return nullptr;
   }
   void* h = PyLong_AsVoidPtr(a[0]);
@@ -541,10 +562,11 @@ PyObject* bind(PyObject*, PyObject* const* a, Py_ssize_t n) {
     PyErr_SetString(PyExc_RuntimeError, "libmqk.so lacks an entry point mqk._front calls");
     return nullptr;
   }
-  for (int i = 1; i < 4; ++i) Py_INCREF(a[i]);
+  for (int i = 1; i < 5; ++i) Py_INCREF(a[i]);
   g_workspaces = a[1];
   g_raw_stream = a[2];
   g_parameter = a[3];
+  g_capturing = a[4];
   g_bound = true;
   Py_RETURN_NONE;
 }
@@ -555,7 +577,7 @@ PyCFunction fast(F f) {
 }
 
 PyMethodDef g_methods[] = {
-    {"bind", fast(bind), METH_FASTCALL, "bind(libmqk handle, workspaces, raw stream accessor, Parameter class)"},
+    {"bind", fast(bind), METH_FASTCALL, "bind(libmqk handle, workspaces, raw stream accessor, Parameter class, capture check)"},
     {"fused", fast(fused), METH_FASTCALL, "fused_qkv_rope of an ordinary call: (q, k, v), a status, or None"},
     {"fused_ex", fast(fused_ex), METH_FASTCALL, "fused_qkv_rope_ex of an ordinary call"},
     {"fused_ex_w4", fast(fused_ex_w4), METH_FASTCALL, "fused_qkv_rope_w4a16_ex of an ordinary call"},

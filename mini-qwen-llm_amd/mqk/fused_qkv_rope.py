@@ -96,10 +96,6 @@ def _rope_tables(cos, sin, D, device, dtype=torch.bfloat16):
     return cos, sin
 
 
-def _no_bytes() -> int:
-    return 0
-
-
 _ENTRIES = {torch.bfloat16: "mqk_fused_qkv_rope_bf16", torch.float16: "mqk_fused_qkv_rope_f16_ws",
             torch.float32: "mqk_fused_qkv_rope_f32"}
 
@@ -163,14 +159,13 @@ def fused_qkv_rope(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), stream)
         _native.check(status, "mqk_fused_qkv_rope_f32")
         return q, k, v
+    entry = _ENTRIES[dtype]
     if dtype == torch.float16:
-        # (no workspace is needed to run: one that cannot grow during capture is passed as it is)
-        entry, least = "mqk_fused_qkv_rope_f16_ws", _no_bytes
         nbytes = int(lib.mqk_fused_qkv_rope_f16_workspace_size(T, H_Q, H_KV, H, D))
+        ws = _native.graph_workspace(device, nbytes) if _native.capturing() else \
+            _native.workspace(device, stream, nbytes)
     else:
-        entry, least = "mqk_fused_qkv_rope_bf16", None
-        nbytes = _native.fused_workspace_bytes(T, H_Q, H_KV, H, D)
-    ws = _native.workspace(device, stream, nbytes, least)
+        ws = _native.workspace(device, stream, _native.fused_workspace_bytes(T, H_Q, H_KV, H, D))
     status = _native.call(
         device, getattr(lib, entry),
         x.data_ptr(), w_q.data_ptr(), w_k.data_ptr(), w_v.data_ptr(),

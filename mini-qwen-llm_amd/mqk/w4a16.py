@@ -307,8 +307,11 @@ def _fused_w4a16(x, q_proj, k_proj, v_proj, q_norm_w, k_norm_w, cos, sin, positi
     lib = _native.library()
     stream = _native.stream_handle(device)
     nbytes = _native.fused_workspace_bytes(T, H_Q, H_KV, H, D, ext, int4=True)
-    ws = _native.workspace(device, stream, nbytes,
-                           lambda: _native.least_workspace_bytes(T, H_Q, H_KV, H, D, ext))
+    if _native.capturing() and nbytes > _native.fused_workspace_bytes(T, H_Q, H_KV, H, D, ext):
+        ws = _native.graph_workspace(device, nbytes)  # (the call unpacks its weights)
+    else:
+        ws = _native.workspace(device, stream, nbytes,
+                               lambda: _native.least_workspace_bytes(T, H_Q, H_KV, H, D, ext))
     flat = [t.data_ptr() for trio in parts for t in trio]
     head = (x.data_ptr(), *flat, group_size, sts[0],
             q_norm_w.data_ptr(), k_norm_w.data_ptr(), cos.data_ptr(), sin.data_ptr(),
