@@ -478,6 +478,9 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     pl.splits = 0;
     base = decode_counter_bytes();
   }
+  if (!pl.v && pl.splits == 0)  // (only pair tiles leave no plan without their workspace)
+    return fail(MQK_ERR_WORKSPACE, "prefill_tile variant %lld needs more workspace than %zu bytes",
+                (long long)g_prefill_tile.load(), workspace ? ws_bytes : size_t(0));
   const size_t scale_off = align_up(base, 256);
   const bool pair = pl.v && is_pair_variant(pl.v->id);
   const size_t need = p.in_gamma ? scale_off + size_t(p.M) * sizeof(float)

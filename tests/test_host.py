@@ -314,6 +314,22 @@ def test_f32_validation(lib):
     assert f(T=-1) == -2
 
 
+@pytest.mark.parametrize("nbytes", [0, 1 << 16, 1 << 17])
+def test_requested_pair_tiles_without_their_workspace(lib, nbytes):
+    """A pair variant set as prefill_tile and a workspace that does not hold its exchange
+    area: an error (before any launch: fake pointers), never a call that computes nothing."""
+    from mqk import _native
+    fake = 1 << 20
+    call = lambda: lib.mqk_fused_qkv_rope_bf16(*[fake] * 8, None, 2048, 2048, 1024, 16, 4, 128, 2048, 1e-6, fake, fake,
+                                               fake, fake if nbytes else None, nbytes, None)
+    _native.set_option("prefill_tile", 24)
+    try:
+        assert lib.mqk_fused_qkv_rope_workspace_size(2048, 16, 4, 1024) > nbytes
+        assert call() == -5  # MQK_ERR_WORKSPACE
+    finally:
+        _native.set_option("prefill_tile", 0)
+
+
 def test_qk_norm_rope_validation(lib):
     fake = 1 << 20
     f = lambda T=4, Hq=2, Hkv=1, D=128, qr=fake: lib.mqk_qk_norm_rope_bf16(
