@@ -351,6 +351,14 @@ size_t plan_region(const Plan& q, int64_t M, int n_tiles) {
   return q.splits > 0 ? decode_workspace_bytes(n_tiles, q.splits, q.passes) : decode_counter_bytes();
 }
 
+// The least of that region with which run_fused still runs a call of this plan: its
+// other plans need none, but a one-block decode launch and requested pair tiles have no
+// other.
+size_t least_region(const Plan& q, int64_t M, int n_tiles) {
+  const bool fixed = q.v ? is_pair_variant(q.v->id) && g_prefill_tile.load() != 0 : M <= 64;
+  return fixed ? plan_region(q, M, n_tiles) : decode_counter_bytes();
+}
+
 // Bytes of normalised rows of a call with an input norm (0: too many, see
 // kNormAheadMaxBytes).
 size_t norm_ahead_bytes(int64_t M, int64_t K) {
@@ -392,9 +400,11 @@ std::unique_lock<std::recursive_mutex> handover_lock(const void* workspace) {
 
 // Common launcher of the fused op (bf16 or int4 weights).  With an input norm
 // (p.in_gamma set, epsilon in_eps), a pre-pass first writes the normalised rows to
-// the workspace after the plan's region, and the plan runs on them; a workspace
-// without that room holds the per-token scales there instead, and the projection
-// kernels normalise what they stage.
+// the workspace's end, and the call without a norm runs on them in what is left of it.  (Its
+// plan there may be another than the size query's, which does not know head_dim 64 or a
+// large cache to exclude pair tiles: it is the plain call's with that workspace.)  A
+// workspace without that room holds the per-token scales after the plan's region instead,
+// and the projection kernels normalise what they stage.
 int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& e, float in_eps,
               void* workspace, size_t ws_bytes, hipStream_t stream, bool allow_pair = true) {
   if (p.M == 0) return ok();
@@ -405,7 +415,7 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     const Plan pl = plan_fused(0, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true,
                                allow_pair && pair_tiles_ok(e));
     const size_t rows = p.in_gamma ? std::max(norm_ahead_bytes(p.M, p.K), align_up(size_t(p.M) * sizeof(float), 256)) : 0;
-    if (epilogue_aligned(e) && off >= align_up(plan_region(pl, p.M, p.n_tiles), 256) + rows) {
+    if (epilogue_aligned(e) && off >= align_up(least_region(pl, p.M, p.n_tiles), 256) + rows) {
       uint16_t* wt = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
       const auto lock = handover_lock(workspace);
       const int st = hip_status(launch_w4_unpack(w, p.n_tiles, p.K, wt, stream), "int4 weight unpack launch");
@@ -418,14 +428,15 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
       return run_fused(0, p, wu, e, in_eps, workspace, off, stream, allow_pair);
     }
   }
-  if (p.in_gamma && workspace && norm_ahead_bytes(p.M, p.K) > 0) {
+  const size_t rows = p.in_gamma && workspace ? norm_ahead_bytes(p.M, p.K) : 0;
+  if (rows > 0 && ws_bytes > rows) {
     // (pair tiles with an input norm are kept to the hidden sizes at which gamma
     // also fits the LDS beside their ring, whichever form the workspace allows)
     const bool pair_lds = tile_dma_lds_bytes(28) + p.K * 2 <= 160 * 1024;
     const bool pairs = pair_lds && pair_tiles_ok(e);
     const Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true, pairs, p.half);
-    const size_t off = align_up(plan_region(pl, p.M, p.n_tiles), 256);
-    if (ws_bytes >= off + norm_ahead_bytes(p.M, p.K)) {
+    const size_t off = (ws_bytes - rows) & ~size_t(255);
+    if (off >= least_region(pl, p.M, p.n_tiles)) {
       uint16_t* xn = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
       const auto lock = handover_lock(workspace);
       const int st = hip_status(launch_row_scale(p.x, p.in_gamma, p.M, p.K, in_eps, nullptr, xn, stream),

@@ -135,3 +135,58 @@ def test_capture_in_a_workspace_of_the_scales_only(device):
         for a, b in zip(out, want):
             assert bool(((a.float() - b.float()).abs() <= 2.0 ** -7 * b.float().abs() + 1e-3).all())
     _native._workspaces.pop((device.index or 0, int(stream.cuda_stream)))
+
+
+@pytest.mark.parametrize("T,hidden,heads,kv,D,int4", [
+    (1100, 3072, 40, 10, 64, False),  # the size query plans pair tiles, the call the split-K launch: ten times the bytes
+    (777, 4096, 64, 16, 64, False), (900, 2048, 48, 24, 64, False), (130, 4096, 64, 16, 64, False), (500, 8448, 20, 5, 128, False),
+    (1000, 4096, 32, 8, 128, False), (300, 2048, 32, 4, 128, False), (40, 1024, 16, 8, 64, False),
+    (777, 4096, 64, 16, 64, True), (130, 1024, 16, 8, 128, True), (1300, 4096, 64, 16, 64, True)])
+def test_rows_are_written_ahead_at_the_queried_size(T, hidden, heads, kv, D, int4, device):
+    """A workspace of exactly the queried bytes holds the normalised rows at its end
+    (before the unpacked weights of a large int4 call), whatever plan the call takes, and
+    the outputs are the plain call's on those rows in what is left of it, bit for bit."""
+    from mqk import _native
+    lib = _native.library()
+    g = torch.Generator(device=device).manual_seed(T + hidden)
+    r = lambda *s: torch.randn(*s, generator=g, device=device)
+    x, gam = (3 * r(T, hidden)).bfloat16(), (1 + 0.3 * r(hidden)).bfloat16()
+    gq, gk = ((1 + 0.1 * r(D)).bfloat16() for _ in range(2))
+    cos, sin = (r(T, D).bfloat16() for _ in range(2))
+    counts = (heads, kv, kv)
+    if int4:
+        w = [t for h in counts for t in
+             (torch.randint(-2**31, 2**31 - 1, (hidden // 8, h * D), generator=g, device=device).int(),
+              (0.005 + 0.015 * torch.rand(hidden // 64, h * D, generator=g, device=device)).half(),
+              torch.randint(-2**31, 2**31 - 1, (hidden // 64, h * D // 8), generator=g, device=device).int())]
+        flat = [t.data_ptr() for t in w] + [64, _native.MQK_SCALE_FP16]
+    else:
+        w = [(0.02 * r(h * D, hidden)).bfloat16() for h in counts]
+        flat = [t.data_ptr() for t in w]
+    ext = _native.FusedExt(in_gamma=gam.data_ptr(), in_eps=1e-6)
+    full = _native.fused_workspace_bytes(T, heads, kv, hidden, D, ext, int4=int4)
+    entry = lib.mqk_fused_qkv_rope_ex_w4a16 if int4 else lib.mqk_fused_qkv_rope_ex_bf16
+
+    def run(rows_in, e, ws, nbytes):
+        out = [torch.zeros(T, h, D, dtype=torch.bfloat16, device=device) for h in counts]
+        st = entry(rows_in.data_ptr(), *flat, gq.data_ptr(), gk.data_ptr(), cos.data_ptr(), sin.data_ptr(), None, T, T,
+                   hidden, heads, kv, D, T, 1e-6, *(o.data_ptr() for o in out), ctypes.byref(e), ws.data_ptr(), nbytes,
+                   int(torch.cuda.current_stream().cuda_stream))
+        _native.check(st, "ex")
+        torch.cuda.synchronize()
+        return out
+
+    ws = torch.zeros(full, dtype=torch.uint8, device=device)
+    out = run(x, ext, ws, full)
+    wbytes = sum(h * D for h in counts) * hidden * 2 if full > _native.fused_workspace_bytes(T, heads, kv, hidden, D, ext) else 0
+    nrows = T * hidden * 2
+    at = (full - wbytes & ~255) - (nrows + 255) // 256 * 256
+    rows = ws[at:at + nrows].view(torch.bfloat16).reshape(T, hidden).clone()
+    y = (x.double() * torch.rsqrt(x.double().square().mean(-1, keepdim=True) + 1e-6)).bfloat16()
+    want = (gam.double() * y.double()).bfloat16()
+    ulps = (rows.view(torch.int16).int() - want.view(torch.int16).int()).abs()
+    assert int(ulps.max()) <= 2 and float((ulps > 0).float().mean()) < 5e-3  # (see test_rows_are_the_rounded_norm)
+    left = at + wbytes  # (the plain call's weights again at the end of what it is given)
+    plain = run(rows, _native.FusedExt(), torch.zeros(left, dtype=torch.uint8, device=device), left)
+    for name, a, b in zip("qkv", out, plain):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), name
