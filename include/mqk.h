@@ -350,8 +350,8 @@ typedef struct mqk_fused_ext {
 } mqk_fused_ext;
 
 /* Workspace bytes of the _ex entry points (the plain size, plus the normalised rows
- * when ext->in_gamma is set, or the per-token scales where the rows would exceed
- * 256 MiB). */
+ * when ext->in_gamma is set, or, where the rows would exceed 256 MiB, the per-token
+ * scales and 64 rows). */
 size_t mqk_fused_qkv_rope_ex_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden,
                                             const mqk_fused_ext* ext);
 

@@ -197,18 +197,19 @@ int plan_tile_split(int64_t M, int64_t K, int n_tiles, const Topology& topo, con
 }
 
 // in_norm: the kernels normalise x themselves (a workspace without room for the
-// normalised rows): whole-head and single-head tiles only.  allow_decode false: a
+// normalised rows): whole-head, single-head and pair tiles only, and a tail of decode
+// rows, few enough to be written ahead.  allow_decode false: a
 // workspace without room for the decode kernel's partials (fp16 only; the other types'
 // entry points require it).
 Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const Topology& topo,
                 bool allow_blocks = true, bool in_norm = false, bool allow_split = true, bool allow_pair = false,
                 int half = 0, bool allow_decode = true) {
-  if (in_norm) allow_decode = allow_blocks = allow_split = allow_pair = false;
+  if (in_norm) allow_blocks = allow_split = false;
   allow_pair = allow_pair && !int4 && aligned && g_pair_tiles.load() != 0;
   Plan pl;
   const int64_t cus = topo.cus;
   if (half) allow_blocks = allow_split = false;  // (fp16: the one-block decode kernel and the tiles)
-  if (use_decode(M) && aligned && allow_decode) {
+  if (use_decode(M) && aligned && allow_decode && !in_norm) {
     pl.splits = decode_splits_for(M, K, n_tiles, int(g_decode_splits.load()), topo.cus, topo.xcds);
     if (pl.splits > 0) {
       pl.tail = M;
@@ -263,7 +264,7 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
   //   launch, e.g. hidden 5120 at T = 384 / 512: 98 us against 119 / 158).
   const TileVariant* hv = nullptr;
   double head_us = 1e30;
-  if (aligned && (M > 64 || !allow_decode) && g_prefill_tile.load() == 0 && g_head_tiles.load() != 0) {
+  if (aligned && (M > 64 || !allow_decode || in_norm) && g_prefill_tile.load() == 0 && g_head_tiles.load() != 0) {
     const int64_t t64 = (M + 63) / 64 * n_tiles, t128 = (M + 127) / 128 * n_tiles;
     const double stages = double(K / 64);
     const bool one64 = t64 <= cus, one128 = t128 <= cus;
@@ -287,7 +288,8 @@ Plan plan_fused(int int4, int64_t M, int64_t K, int n_tiles, bool aligned, const
     for (int i = 0; i < tile_variant_count(); ++i)
       if (tile_variant(i)->id == 26) pv = tile_variant(i);
     const int64_t wgs = pv ? tile_count(*pv, M, n_tiles) : 0;
-    if (pv && 2 * wgs > cus && wgs <= cus && wgs / 2 <= kSplitMaxTiles) {
+    if (pv && 2 * wgs > cus && wgs <= cus && wgs / 2 <= kSplitMaxTiles &&
+        !(in_norm && tile_dma_lds_bytes(26) + K * 2 > 160 * 1024)) {
       pair_us = 15.0 + double(K / 64) * (0.465 + 0.001 * double(wgs));
     } else {
       pv = nullptr;
@@ -366,6 +368,13 @@ size_t norm_ahead_bytes(int64_t M, int64_t K) {
   return n <= kNormAheadMaxBytes ? n : 0;
 }
 
+// Workspace bytes of the input norm beside a plan's region: the rows, or, where they are
+// too many, the per-token scales and the rows of a decode tail.
+size_t input_norm_bytes(int64_t M, int64_t K) {
+  const size_t rows = norm_ahead_bytes(M, K);
+  return rows > 0 ? rows : align_up(size_t(M) * sizeof(float), 256) + align_up(size_t(64) * size_t(K) * 2, 256);
+}
+
 // int4 calls whose weights are unpacked to bf16 in the workspace first
 // (w4_unpack.hip), and the bytes that takes (0: the int4 kernels run the call).  From
 // kUnpackFlops on, measured on MI355X: hidden 4096, 32 / 8 heads T = 1536 135 -> 104 us,
@@ -414,7 +423,7 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     const size_t off = (ws_bytes - wb) & ~size_t(255);
     const Plan pl = plan_fused(0, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true,
                                allow_pair && pair_tiles_ok(e));
-    const size_t rows = p.in_gamma ? std::max(norm_ahead_bytes(p.M, p.K), align_up(size_t(p.M) * sizeof(float), 256)) : 0;
+    const size_t rows = p.in_gamma ? input_norm_bytes(p.M, p.K) : 0;
     if (epilogue_aligned(e) && off >= align_up(least_region(pl, p.M, p.n_tiles), 256) + rows) {
       uint16_t* wt = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
       const auto lock = handover_lock(workspace);
@@ -430,8 +439,9 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
   }
   const size_t rows = p.in_gamma && workspace ? norm_ahead_bytes(p.M, p.K) : 0;
   if (rows > 0 && ws_bytes > rows) {
-    // (pair tiles with an input norm are kept to the hidden sizes at which gamma
-    // also fits the LDS beside their ring, whichever form the workspace allows)
+    // (pair tiles with an input norm are kept to the hidden sizes at which gamma fits the
+    // LDS beside their ring, so that a call takes the same tiles whichever form its
+    // workspace allows)
     const bool pair_lds = tile_dma_lds_bytes(28) + p.K * 2 <= 160 * 1024;
     const bool pairs = pair_lds && pair_tiles_ok(e);
     const Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true, pairs, p.half);
@@ -457,16 +467,25 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
                 (long long)g_prefill_tile.load(), p.n_tiles, int4 ? ", int4 weights" : "");
   auto region = [&](const Plan& q) { return plan_region(q, p.M, p.n_tiles); };
   size_t base = region(pl);
-  // bytes the plan needs: the decode (or split-tile) region, then (input norm) the per-token scales
+  // bytes the plan needs: the decode (or split-tile) region, then (input norm) the
+  // per-token scales and the normalised rows of the decode tail
   const size_t scale_bytes = p.in_gamma ? align_up(size_t(p.M) * sizeof(float), 256) : 0;
-  auto fits = [&](size_t b) { return workspace && ws_bytes >= align_up(b, 256) + scale_bytes; };
+  auto tail_bytes = [&]() { return p.in_gamma ? size_t(pl.tail) * size_t(p.K) * 2 : 0; };
+  auto fits = [&](size_t b) { return workspace && ws_bytes >= align_up(b, 256) + scale_bytes + tail_bytes(); };
+  if (p.in_gamma && pl.tail > 0 && !fits(base)) {
+    pl.tail = 0;  // (before the pair tiles are given up)
+    pl.splits = 0;
+    base = region(pl);
+  }
   if (pl.ksplit > 0 && (!fits(base) || !epilogue_aligned(e))) {
     // a workspace sized without the split-K tile launch (or operands it cannot take): plan without it
     pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, false, pair_ok, p.half);
     base = region(pl);
   }
-  if (pl.v && is_pair_variant(pl.v->id) && !fits(base)) {
-    // a workspace sized without the pair tiles' exchange area: plan without them
+  if (pl.v && is_pair_variant(pl.v->id) &&
+      (!fits(base) || (p.in_gamma && tile_dma_lds_bytes(pl.v->id) + p.K * 2 > 160 * 1024))) {
+    // a workspace sized without the pair tiles' exchange area, or an input norm whose
+    // gamma does not fit the LDS beside their ring: plan without them
     pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, p.in_gamma != nullptr, false, false, p.half);
     base = region(pl);
   }
@@ -489,12 +508,16 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     pl.splits = 0;
     base = decode_counter_bytes();
   }
-  if (!pl.v && pl.splits == 0)  // (only pair tiles leave no plan without their workspace)
+  if (!pl.v && pl.splits == 0) {  // (requested pair tiles that cannot run leave no other plan)
+    if (p.in_gamma && fits(0))
+      return fail(MQK_ERR_BAD_OPTION, "prefill_tile variant %lld cannot run this input norm (hidden %lld)",
+                  (long long)g_prefill_tile.load(), (long long)p.K);
     return fail(MQK_ERR_WORKSPACE, "prefill_tile variant %lld needs more workspace than %zu bytes",
                 (long long)g_prefill_tile.load(), workspace ? ws_bytes : size_t(0));
+  }
   const size_t scale_off = align_up(base, 256);
   const bool pair = pl.v && is_pair_variant(pl.v->id);
-  const size_t need = p.in_gamma ? scale_off + size_t(p.M) * sizeof(float)
+  const size_t need = p.in_gamma ? scale_off + (pl.tail > 0 ? scale_bytes + tail_bytes() : size_t(p.M) * sizeof(float))
                                  : ((pl.splits > 0 || pl.ksplit > 0 || pair) ? base : 0);
   if (need > 0 && (!workspace || ws_bytes < need))
     return fail(MQK_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given%s", need, ws_bytes,
@@ -507,6 +530,14 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
                               "input norm pre-pass launch");
     if (st != MQK_OK) return st;
     p.in_scale = scale;
+  }
+  uint16_t* tail_rows = nullptr;  // (input norm) the normalised rows of the decode tail
+  if (p.in_gamma && pl.tail > 0) {
+    tail_rows = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + scale_off + scale_bytes);
+    const int st = hip_status(launch_row_scale(p.x + (p.M - pl.tail) * p.K, p.in_gamma, pl.tail, p.K, in_eps, nullptr,
+                                               tail_rows, stream),
+                              "input norm pre-pass launch (tail)");
+    if (st != MQK_OK) return st;
   }
   if (pl.ksplit > 0)
     return hip_status(launch_tile_dma_split(pl.v->id, p, w, e, pl.ksplit, g_decode_force_recompute,
@@ -537,7 +568,11 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     ProblemArgs pt = p;
     pt.M = std::min<int64_t>(rows_per_launch, p.M - t0);
     pt.x = p.x + t0 * p.K;
-    if (p.in_scale) pt.in_scale = p.in_scale + t0;
+    if (tail_rows) {  // (at most 64 rows, one launch)
+      pt.x = tail_rows;
+      pt.in_gamma = nullptr;
+      pt.in_scale = nullptr;
+    }
     EpilogueArgs et = e;
     et.t0 = t0;
     auto shift = [&](uint16_t* ptr, int heads) { return ptr ? ptr + t0 * heads * kHeadDim : ptr; };
@@ -620,8 +655,7 @@ size_t mqk_fused_qkv_rope_workspace_size_hd(int64_t T, int Hq, int Hkv, int64_t 
       const size_t m = plan_bytes(int4, T, hidden, tiles, topo, true);
       // (with the fused input RMSNorm: that plan, then the normalised rows or the scales)
       if (m != ~size_t(0))
-        n = std::max(n, align_up(m > 0 ? m : decode_counter_bytes(), 256) +
-                            std::max(norm_ahead_bytes(T, hidden), align_up(size_t(T) * sizeof(float), 256)));
+        n = std::max(n, align_up(m > 0 ? m : decode_counter_bytes(), 256) + input_norm_bytes(T, hidden));
     }
   for (int int4 = 0; int4 < 2; ++int4)
     for (int h : {Hq, Hkv}) {
@@ -635,10 +669,8 @@ size_t mqk_fused_qkv_rope_workspace_size_hd(int64_t T, int Hq, int Hkv, int64_t 
 size_t mqk_fused_qkv_rope_ex_workspace_size(int64_t T, int Hq, int Hkv, int64_t hidden,
                                             const mqk_fused_ext* ext) {
   size_t n = mqk_fused_qkv_rope_workspace_size(T, Hq, Hkv, hidden);
-  if (ext && ext->in_gamma && T > 0 && hidden > 0) {
-    const size_t rows = norm_ahead_bytes(T, hidden);
-    n = align_up(n > 0 ? n : decode_counter_bytes(), 256) + (rows > 0 ? rows : align_up(size_t(T) * sizeof(float), 256));
-  }
+  if (ext && ext->in_gamma && T > 0 && hidden > 0)
+    n = align_up(n > 0 ? n : decode_counter_bytes(), 256) + input_norm_bytes(T, hidden);
   return n;
 }
 

@@ -190,3 +190,62 @@ def test_rows_are_written_ahead_at_the_queried_size(T, hidden, heads, kv, D, int
     plain = run(rows, _native.FusedExt(), torch.zeros(left, dtype=torch.uint8, device=device), left)
     for name, a, b in zip("qkv", out, plain):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), name
+
+
+def test_more_rows_than_are_written_ahead(device):
+    """Above 256 MiB of rows the projection kernels normalise what they stage, with the
+    plain plan's pair tiles and the rows past its last whole tile on the decode kernel
+    (which reads those few rows ahead).  Every row must be the row of a call that writes
+    it ahead: the same bits on the tiles, one bf16 ulp on the decode rows, whose sums are
+    split differently."""
+    import mqk
+    from conftest import launched_kernels
+    T, hidden, Hq, Hkv, tail = 32768 + 22, 5120, 9, 3, 22
+    g = torch.Generator(device=device).manual_seed(3)
+    w = [(0.02 * torch.randn(h * D, hidden, generator=g, device=device)).bfloat16() for h in (Hq, Hkv, Hkv)]
+    one = torch.ones(D, dtype=torch.bfloat16, device=device)
+    cos, sin = (torch.randn(4096, D, generator=g, device=device).bfloat16() for _ in range(2))
+    gam = (1 + 0.3 * torch.randn(hidden, generator=g, device=device)).bfloat16()
+    x = torch.randn(1, T, hidden, generator=g, device=device).bfloat16()
+    pos = torch.randint(0, 4096, (T,), generator=g, device=device).int()
+    call = lambda a, b: mqk.fused_qkv_rope_ex(x[:, a:b], *w, one, one, cos, sin, pos[a:b], input_norm_w=gam)
+    assert launched_kernels(lambda: call(0, T)) == ["row_scale", "row_scale", "tile_pair", "decode"]
+    out = call(0, T)
+    for a in range(0, T, 16384):
+        b = min(a + 16384, T)
+        for name, o, r in zip("qkv", out, call(a, b)):
+            o = o[:, a:b]
+            if b == T:
+                o, r = o[:, -tail:].float(), r[:, -tail:].float()
+                assert bool(((o - r).abs() <= 2.0 ** -7 * r.abs() + 1e-3).all()), name
+            else:
+                assert torch.equal(o.view(torch.int16), r.view(torch.int16)), name
+    mqk.set_option("prefill_tile", 25)  # (the planned pair tiles: accepted by name too)
+    try:
+        tiles = call(0, T)
+        torch.cuda.synchronize()
+    finally:
+        mqk.set_option("prefill_tile", 0)
+    for name, o, r in zip("qkv", tiles, out):
+        assert torch.equal(o[:, :-tail].view(torch.int16), r[:, :-tail].view(torch.int16)), name
+    torch.cuda.synchronize()
+    mqk.release_workspaces(retired_only=False)
+
+
+@pytest.mark.parametrize("tile", [16, 24, 25])
+@pytest.mark.parametrize("T", [2048, 2078])
+def test_both_forms_agree_on_one_kernel(T, tile, device):
+    """With one tile variant requested, the call with rows written ahead and the one with
+    their scales only give the same bits (but for rows that go to the decode kernel)."""
+    import mqk
+    Hq, Hkv = (20, 5) if tile == 25 else (32, 8)
+    mqk.set_option("prefill_tile", tile)
+    mqk.set_option("tail_split", 0)
+    try:
+        run, full, least = _call(T, 1024, Hq, Hkv, False, 5, device)
+        (ahead, _), (staged, _) = run(full), run(least)
+    finally:
+        mqk.set_option("prefill_tile", 0)
+        mqk.set_option("tail_split", 1)
+    for name, a, b in zip("qkv", ahead, staged):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), name
