@@ -375,6 +375,11 @@ size_t input_norm_bytes(int64_t M, int64_t K) {
   return rows > 0 ? rows : align_up(size_t(M) * sizeof(float), 256) + align_up(size_t(64) * size_t(K) * 2, 256);
 }
 
+// The least workspace of a call with an input norm whose plan without one is q, M <= 64.
+size_t input_norm_least(const Plan& q, int64_t M, int n_tiles) {
+  return align_up(plan_region(q, M, n_tiles), 256) + size_t(M) * sizeof(float);
+}
+
 // int4 calls whose weights are unpacked to bf16 in the workspace first
 // (w4_unpack.hip), and the bytes that takes (0: the int4 kernels run the call).  From
 // kUnpackFlops on, measured on MI355X: hidden 4096, 32 / 8 heads T = 1536 135 -> 104 us,
@@ -413,9 +418,13 @@ std::unique_lock<std::recursive_mutex> handover_lock(const void* workspace) {
 // plan there may be another than the size query's, which does not know head_dim 64 or a
 // large cache to exclude pair tiles: it is the plain call's with that workspace.)  A
 // workspace without that room holds the per-token scales after the plan's region instead,
-// and the projection kernels normalise what they stage.
+// and the projection kernels normalise what they stage.  The decode kernel has no such
+// form: with room for the plan's region and the scales only, it runs with fewer splits
+// than planned (decode_splits of the inner call), whose partials leave room for the rows
+// (hidden 4096, 32 / 8 heads, T = 8 19.6 us, T = 64 23.4, against 18.4 and 22.1 with all
+// splits, and 50.3 and 50.9 for tiles that normalise).
 int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& e, float in_eps,
-              void* workspace, size_t ws_bytes, hipStream_t stream, bool allow_pair = true) {
+              void* workspace, size_t ws_bytes, hipStream_t stream, bool allow_pair = true, int decode_splits = 0) {
   if (p.M == 0) return ok();
   const Topology topo = device_topology();
   if (const size_t wb = int4 && e.qkv && workspace ? unpack_bytes(p.M, p.K, p.n_tiles) : 0; wb > 0 && ws_bytes > wb) {
@@ -446,7 +455,16 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
     const bool pairs = pair_lds && pair_tiles_ok(e);
     const Plan pl = plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo, true, false, true, pairs, p.half);
     const size_t off = (ws_bytes - rows) & ~size_t(255);
-    if (off >= least_region(pl, p.M, p.n_tiles)) {
+    bool room = off >= least_region(pl, p.M, p.n_tiles);
+    int splits = 0;
+    if (!room && !pl.v && p.M <= 64 && ws_bytes >= input_norm_least(pl, p.M, p.n_tiles))
+      for (int s = pl.splits - 1; s >= 1 && !room; --s)
+        if (decode_splits_for(p.M, p.K, p.n_tiles, s, topo.cus, topo.xcds) == s &&
+            off >= decode_workspace_bytes(p.n_tiles, s)) {
+          room = true;
+          splits = s;
+        }
+    if (room) {
       uint16_t* xn = reinterpret_cast<uint16_t*>(static_cast<char*>(workspace) + off);
       const auto lock = handover_lock(workspace);
       const int st = hip_status(launch_row_scale(p.x, p.in_gamma, p.M, p.K, in_eps, nullptr, xn, stream),
@@ -454,7 +472,7 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
       if (st != MQK_OK) return st;
       p.x = xn;
       p.in_gamma = nullptr;
-      return run_fused(int4, p, w, e, 0.f, workspace, off, stream, pair_lds);
+      return run_fused(int4, p, w, e, 0.f, workspace, off, stream, pair_lds, splits);
     }
   }
   p.cus = topo.cus;
@@ -465,6 +483,7 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
   if (!pl.v && pl.splits == 0)
     return fail(MQK_ERR_BAD_OPTION, "prefill_tile variant %lld cannot run this problem (%d heads%s)",
                 (long long)g_prefill_tile.load(), p.n_tiles, int4 ? ", int4 weights" : "");
+  if (decode_splits > 0 && !pl.v) pl.splits = decode_splits;
   auto region = [&](const Plan& q) { return plan_region(q, p.M, p.n_tiles); };
   size_t base = region(pl);
   // bytes the plan needs: the decode (or split-tile) region, then (input norm) the
@@ -517,8 +536,10 @@ int run_fused(int int4, ProblemArgs p, const WeightArgs& w, const EpilogueArgs& 
   }
   const size_t scale_off = align_up(base, 256);
   const bool pair = pl.v && is_pair_variant(pl.v->id);
-  const size_t need = p.in_gamma ? scale_off + (pl.tail > 0 ? scale_bytes + tail_bytes() : size_t(p.M) * sizeof(float))
-                                 : ((pl.splits > 0 || pl.ksplit > 0 || pair) ? base : 0);
+  size_t need = p.in_gamma ? scale_off + (pl.tail > 0 ? scale_bytes + tail_bytes() : size_t(p.M) * sizeof(float))
+                           : ((pl.splits > 0 || pl.ksplit > 0 || pair) ? base : 0);
+  if (p.in_gamma && p.M <= 64)  // (at decode sizes the plain size and the scales are the least)
+    need = std::max(need, input_norm_least(plan_fused(int4, p.M, p.K, p.n_tiles, epilogue_aligned(e), topo), p.M, p.n_tiles));
   if (need > 0 && (!workspace || ws_bytes < need))
     return fail(MQK_ERR_WORKSPACE, "workspace of %zu bytes needed, %zu given%s", need, ws_bytes,
                 workspace ? "" : " (NULL)");
@@ -619,6 +640,13 @@ static size_t plan_bytes(int int4, int64_t M, int64_t K, int tiles, const Topolo
   if (pl.ksplit > 0) n = std::max(n, kDecodeCounterBytes + tile_split_part_bytes(pl.v->id, M, tiles, pl.ksplit));
   if (pl.v && is_pair_variant(pl.v->id)) n = std::max(n, pair_tile_workspace_bytes(pl.v->id, M - pl.tail, tiles));
   return n;
+}
+
+// ... the q/k/v launch of the generic head sizes, with the scales of an input norm.
+static size_t any_d_need(int int4, int64_t T, int64_t hidden, int tiles, const Topology& topo, bool in_norm) {
+  const size_t n = plan_bytes(int4, T, hidden, tiles, topo, true);
+  if (!in_norm || n == ~size_t(0)) return n;
+  return align_up(n > 0 ? n : decode_counter_bytes(), 256) + align_up(size_t(T) * sizeof(float), 256);
 }
 
 static size_t plain_plan_bytes(int int4, int64_t M, int64_t K, int tiles, const Topology& topo) {
@@ -831,9 +859,7 @@ static int fused_bf16_any_d(const mqk_bf16* x, const mqk_bf16* w_q, const mqk_bf
     // as projected (qkv 2), when the workspace holds what that plan needs
     const bool in_norm = ext && ext->in_gamma;
     const int tiles = int((nq + 2 * nkv) / kHeadDim);
-    // (with the input norm the launch takes any workspace that holds its scales)
-    const size_t need = in_norm ? align_up(decode_counter_bytes(), 256) + align_up(size_t(T) * sizeof(float), 256)
-                                : plan_bytes(0, T, hidden, tiles, topo, true);
+    const size_t need = any_d_need(0, T, hidden, tiles, topo, in_norm);
     const bool fits = tiles <= kMaxTiles && need != ~size_t(0) && (need == 0 || (workspace && need <= ws_bytes));
     if (fits) {
       ProblemArgs pr{x, T, hidden, tiles};
@@ -1340,8 +1366,7 @@ static int fused_w4a16_impl(const mqk_bf16* x, const int32_t* qw_q, const void* 
             MQK_OK)
           return st;
       const int tiles = int((nq + 2 * nkv) / kHeadDim);
-      const size_t need = in_norm ? align_up(decode_counter_bytes(), 256) + align_up(size_t(T) * sizeof(float), 256)
-                                  : plan_bytes(1, T, hidden, tiles, topo, true);
+      const size_t need = any_d_need(1, T, hidden, tiles, topo, in_norm);
       if (tiles <= kMaxTiles && need != ~size_t(0) && (need == 0 || (workspace && need <= ws_bytes))) {
         ProblemArgs pr{x, T, hidden, tiles};
         pr.in_gamma = in_norm ? ext->in_gamma : nullptr;

@@ -330,6 +330,28 @@ def test_requested_pair_tiles_without_their_workspace(lib, nbytes):
         _native.set_option("prefill_tile", 0)
 
 
+@pytest.mark.parametrize("int4", [False, True])
+def test_input_norm_workspace_below_the_least(lib, int4):
+    """Decode sizes with an input norm need the plain size and T floats, other head sizes
+    of the W4A16 front their plan's: a byte less is refused before any launch (fake
+    pointers)."""
+    import ctypes
+    from mqk import _native
+    fake, hidden, Hq, Hkv = 1 << 20, 4096, 32, 8
+    ext = _native.FusedExt(in_gamma=fake, in_eps=1e-6)
+    entry = lib.mqk_fused_qkv_rope_ex_w4a16 if int4 else lib.mqk_fused_qkv_rope_ex_bf16
+
+    def call(T, D, nbytes):
+        w = [fake] * 9 + [128, _native.MQK_SCALE_FP16] if int4 else [fake] * 3
+        return entry(fake, *w, fake, fake, fake, fake, None, T, T, hidden, Hq, Hkv, D, T, 1e-6, fake, fake, fake,
+                     ctypes.byref(ext), fake, nbytes, None)
+    for T in (1, 8, 64):
+        plain = int(lib.mqk_fused_qkv_rope_workspace_size(T, Hq, Hkv, hidden))
+        assert call(T, 128, plain + 4 * T - 1) == -5  # MQK_ERR_WORKSPACE
+    if int4:
+        assert call(8, 96, _native._COUNTER_BYTES + 4096) == -3  # MQK_ERR_UNSUPPORTED
+
+
 def test_qk_norm_rope_validation(lib):
     fake = 1 << 20
     f = lambda T=4, Hq=2, Hkv=1, D=128, qr=fake: lib.mqk_qk_norm_rope_bf16(

@@ -249,3 +249,17 @@ def test_both_forms_agree_on_one_kernel(T, tile, device):
         mqk.set_option("tail_split", 1)
     for name, a, b in zip("qkv", ahead, staged):
         assert torch.equal(a.view(torch.int16), b.view(torch.int16)), name
+
+
+@pytest.mark.parametrize("T,hidden,Hq,Hkv,int4", [(1, 1024, 16, 8, False), (16, 4096, 32, 8, False),
+                                                  (64, 4096, 32, 8, False), (24, 5120, 40, 8, False),
+                                                  (8, 4096, 32, 8, True), (64, 2048, 32, 4, True)])
+def test_decode_with_the_least_workspace(T, hidden, Hq, Hkv, int4, device):
+    """Decode sizes in a workspace of the plain size and the scales: still the decode
+    kernel, on rows written ahead beside the partials of fewer splits."""
+    from conftest import launched_kernels
+    run, full, least = _call(T, hidden, Hq, Hkv, int4, 11 + T, device)
+    assert launched_kernels(lambda: run(least)) == ["row_scale", "decode"]
+    for name, a, b in zip("qkv", run(full)[0], run(least)[0]):
+        a, b = a.float(), b.float()
+        assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 1e-3 * b.square().mean().sqrt().clamp(min=1.0)).all()), name
