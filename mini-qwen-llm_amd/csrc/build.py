@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import argparse
 import concurrent.futures as cf
+import importlib.util
 import os
 import re
 import shutil
@@ -109,7 +110,11 @@ def _compile(src: str, verbose: bool, incremental: bool = False) -> Path:
 
 
 def _build_front(verbose: bool, incremental: bool) -> None:
-    """The CPython extension (host code only, against the installed torch)."""
+    """The CPython extension (host code only, against the installed torch; without torch
+    there is no package to extend, and only the library is built)."""
+    if importlib.util.find_spec("torch") is None:
+        print("torch is not installed: mqk._front is not built", flush=True)
+        return
     if incremental and FRONT.exists() and all(
             d.stat().st_mtime < FRONT.stat().st_mtime
             for d in (FRONT_SRC, CSRC.parent.parent / "include" / "mqk.h", Path(__file__))):
@@ -126,7 +131,8 @@ def _build_front(verbose: bool, incremental: bool) -> None:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"front.cpp failed:\n{res.stdout}{res.stderr}")
+        FRONT.unlink(missing_ok=True)  # (an older one need not match the library)
+        raise RuntimeError(f"front.cpp failed (libmqk.so, which does not need it, is built):\n{res.stdout}{res.stderr}")
     os.replace(tmp, FRONT)
 
 
@@ -135,7 +141,12 @@ def build(verbose: bool = False, incremental: bool = False) -> Path:
     with cf.ThreadPoolExecutor(max_workers=min(len(SOURCES) + 1, os.cpu_count() or 1)) as ex:
         front = ex.submit(_build_front, verbose, incremental)
         objs = list(ex.map(lambda s: _compile(s, verbose, incremental), SOURCES))
-        front.result()
+    _link(objs, verbose)
+    front.result()
+    return OUT
+
+
+def _link(objs: list, verbose: bool) -> None:
     tmp = OUT.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     if verbose:
@@ -144,7 +155,6 @@ def build(verbose: bool = False, incremental: bool = False) -> Path:
     if res.returncode != 0:
         raise RuntimeError("link failed:\n" + _filter(res.stdout + res.stderr))
     os.replace(tmp, OUT)
-    return OUT
 
 
 def main(argv=None) -> int:

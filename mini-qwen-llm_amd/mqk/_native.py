@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 from pathlib import Path
 
 import torch  # (imported before the HIP library is mapped)
@@ -208,8 +209,10 @@ def front():
         if _front is None and not _front_absent:
             try:
                 from . import _front as ext
-            except ImportError:
+            except ImportError as exc:
                 ext = None
+                warnings.warn(f"mqk._front is not there ({exc}): build it with csrc/build.py, or every call's checks "
+                              "run in Python, 5 to 20 us slower", RuntimeWarning, stacklevel=3)
             if ext is None or _raw_stream is None:
                 _front_absent = True
             else:
