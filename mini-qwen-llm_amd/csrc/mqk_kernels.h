@@ -101,7 +101,8 @@ const TileVariant* tile_variant(int index);
 // Picks a variant for the problem (id 0 = automatic).
 // allow_pair: the pair-tile variants (24-28) may be chosen (bf16 q/k/v outputs
 // with head_dim 128 and a workspace for their exchange).
-// half: fp16 elements (a requested variant without an fp16 form counts as automatic).
+// half: fp16 elements (a requested variant that cannot run the call in fp16 counts as
+// automatic: the request is about the bf16 and int4 tiles, and fp16 calls never failed for it).
 const TileVariant* choose_tile_variant(int requested_id, int64_t M, int n_tiles, int int4, int cus,
                                        bool allow_pair = false, int half = 0);
 inline bool fp16_variant(int id) {

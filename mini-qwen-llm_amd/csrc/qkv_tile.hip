@@ -462,14 +462,14 @@ int64_t tile_count(const TileVariant& v, int64_t M, int n_tiles) {
 
 const TileVariant* choose_tile_variant(int requested_id, int64_t M, int n_tiles, int int4, int cus_, bool allow_pair,
                                        int half) {
-  if (half && !fp16_variant(requested_id)) requested_id = 0;
   // (a pair launch has one exchange word per pair in the workspace's kSplitMaxTiles lines)
   auto pair_fits = [&](const TileVariant& v) { return allow_pair && tile_count(v, M, n_tiles) / 2 <= kSplitMaxTiles; };
   if (requested_id > 0) {
     const TileVariant* v = find_variant(requested_id);
-    if (!v || n_tiles % v->hpt != 0 || !supports(*v, int4) || (is_pair_variant(v->id) && !pair_fits(*v)))
-      return nullptr;
-    return v;
+    const bool runs = v && n_tiles % v->hpt == 0 && supports(*v, int4) && (!is_pair_variant(v->id) || pair_fits(*v)) &&
+                      (!half || fp16_variant(v->id));
+    if (runs) return v;
+    if (!half) return nullptr;
   }
   // Score = relative per-tile speed (measured on MI355X) x fraction of the last
   // round of workgroups that is busy, assuming one workgroup per CU at a time

@@ -111,3 +111,32 @@ def test_f16_large_values_saturate_like_a_cast(device):
     ref = _exact(*args, None, 128)[2].half()
     assert bool(torch.isinf(out[2][0, 3]).all()) and bool(torch.isinf(ref[3]).all())
     assert bool(torch.isfinite(out[2][0, [0, 2, 4, 69]]).all())
+
+
+@pytest.mark.parametrize("tile", [1, 16, 18, 24, 25, 28, 31])
+def test_a_requested_variant_never_refuses_fp16(tile, device):
+    """prefill_tile names a bf16 or int4 tile: an fp16 call whose head count, workspace or
+    element type that variant does not take runs the automatic choice (the same bits: the
+    tiles sum in one order)."""
+    import mqk
+    from mqk import _native
+    T, hidden, Hq, Hkv = 200, 256, 3, 1  # (5 blocks: whole tiles for 20, 21, 25 and 27 only)
+    g = torch.Generator(device=device).manual_seed(tile)
+    r = lambda *s: torch.randn(*s, generator=g, device=device).half()
+    args = (r(1, T, hidden), *(0.05 * r(h * 128, hidden) for h in (Hq, Hkv, Hkv)), 1 + 0.1 * r(128), 1 + 0.1 * r(128),
+            r(T, 128), r(T, 128))
+    lib = _native.library()
+    out = [torch.zeros(T, h, 128, dtype=torch.float16, device=device) for h in (Hq, Hkv, Hkv)]
+    want = mqk.fused_qkv_rope(*args)
+    old = mqk.get_option("prefill_tile")
+    mqk.set_option("prefill_tile", tile)
+    try:
+        got = mqk.fused_qkv_rope(*args)
+        st = lib.mqk_fused_qkv_rope_f16(*(t.data_ptr() for t in args), None, T, T, hidden, Hq, Hkv, 128, T, 1e-6,
+                                        *(o.data_ptr() for o in out), int(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+    finally:
+        mqk.set_option("prefill_tile", old)
+    _native.check(st, "f16")
+    for a, b, c in zip(got, want, out):
+        assert torch.equal(a, b) and torch.equal(c.reshape(b.shape), b)
