@@ -9,15 +9,17 @@
 // critical path of every stage: measured on MI355X (hidden 4096, 32 / 8 heads,
 // one call, without -> with the rows written ahead) T = 24 25.3 -> 22.4 us, T = 777
 // 71.8 -> 58.8 us, T = 4096 220 -> 194 us; int4 weights T = 777 238 -> 81 us, T = 4096
-// 356 -> 280 us (the plain call: 18.2 / 52.1 / 180 and 75 / 267 us).  A smaller workspace (or more than kNormAheadMaxBytes of rows)
-// gets the scales only, and the projection kernels apply them as they stage
-// their x tiles (input_norm8): the same bits.
+// 356 -> 280 us (the plain call: 18.2 / 52.1 / 180 and 75 / 267 us; T = 24 has since
+// become 20.3 us with the decode kernel's 32-row blocks).  A workspace without room for
+// the rows (or more than kNormAheadMaxBytes of them) gets the scales only, and the tile
+// kernels apply them as they stage their x tiles (input_norm8): the same bits from the
+// same tiles.
 //
 // One wave per token row, bound by latency at decode sizes and by the copy at large
 // T: 16-byte loads, up to 4096 or 8192 of a row's elements and their gammas in flight
 // and held (HELD = 8 or 16 chunks per lane; longer rows are read again for the second
-// pass, from the L2), fp32 sum of squares, 64-lane butterfly.  Rows get a workgroup each until there are enough of
-// them to fill the CUs with four per workgroup.
+// pass, from the L2), fp32 sum of squares, 64-lane butterfly.  Rows get a workgroup each
+// until there are enough of them to fill the CUs with four per workgroup.
 #include "mqk_device.h"
 #include "mqk_kernels.h"
 

@@ -1014,8 +1014,8 @@ static int fused_f32_impl(bool half, const void* x, const void* w_q, const void*
   if (half && hidden % kBK == 0 && aligned16(q_gamma) && aligned16(k_gamma) && aligned16(cos) && aligned16(sin)) {
     // fp16 with whole 64-k stages and 16-byte table rows: the pipelined tile kernels
     // (one call at hidden 4096, 32 / 8 heads on MI355X: T = 1 50.7 us in the kernel
-    // below, 29.8 here; T = 2048 306 and 102).  Other hidden sizes (multiples of 32) and
-    // unaligned tables stay below.
+    // below, 15.5 here, or 29.8 without a workspace for the decode kernel; T = 2048 306
+    // and 102).  Other hidden sizes (multiples of 32) and unaligned tables stay below.
     auto u = [](const void* ptr) { return static_cast<const uint16_t*>(ptr); };
     auto o = [](void* ptr) { return static_cast<uint16_t*>(ptr); };
     ProblemArgs p{u(x), T, hidden, Hq + 2 * Hkv};

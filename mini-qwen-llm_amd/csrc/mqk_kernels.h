@@ -154,7 +154,7 @@ hipError_t launch_tile_dma_w4(int id, const ProblemArgs& p, const WeightArgs& w,
 // Split-K decode kernel for T <= 64.  decode_splits_for returns 0 when no
 // valid split count exists (each split covers at most 16 64-wide k tiles);
 // the caller then uses the tile kernel.
-// LDS bytes (static) of pipelined tile variant id (10..32); 0 for other ids.
+// LDS bytes (static) of pipelined tile variant id (10..35); 0 for other ids.
 int tile_dma_lds_bytes(int id);
 
 // Input RMSNorm pre-pass over x [M, K] bf16 (K <= 16384): with sc[m] =
@@ -163,7 +163,7 @@ int tile_dma_lds_bytes(int id);
 hipError_t launch_row_scale(const uint16_t* x, const uint16_t* gamma, int64_t M, int64_t K, float eps, float* scale,
                             uint16_t* out, hipStream_t stream);
 // Most bytes of normalised rows a call keeps in its workspace; larger calls keep
-// the per-token scales only (so that one long prefill does not leave gigabytes of
+// the per-token scales, and the rows of a decode tail, only (so that one long prefill does not leave gigabytes of
 // workspace behind).
 constexpr size_t kNormAheadMaxBytes = size_t(256) << 20;
 

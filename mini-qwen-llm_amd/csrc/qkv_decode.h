@@ -690,7 +690,7 @@ __device__ __forceinline__ void run_split_multi(const ProblemArgs& p, const Weig
     f32x4_t acc[4];
     zero_acc(acc);
     // this block's x slice in the same LDS once every wave is done with it (the
-    // previous block's MFMAs or a finish); the normalising gamma stays in LDS.
+    // previous block's MFMAs or a finish).
     // Once its first tiles have landed, so have the previous block's partial
     // stores (issued earlier): then that block's arrival is counted and the
     // counter of the oldest noted block read; both values are used after this

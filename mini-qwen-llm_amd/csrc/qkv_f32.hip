@@ -87,7 +87,8 @@ __device__ __forceinline__ void finish_rows(const F32Args& a, const float* ep, i
   }
 }
 
-// The fp32 kernel.  Its bound at T = 128, hidden 1024, 16 / 8 heads is the fp32 matrix
+// The fp32 kernel (tiles of 32 rows and more; 16-row tiles: F32Narrow).  Its bound at
+// T = 128, hidden 1024, 16 / 8 heads is the fp32 matrix
 // core (6.8 us at 256 operations a clock and CU); the weights, 16 MB, take 3.3 us.  So
 // nothing is allowed between the MFMAs but their operands:
 //   * a weight element is used by one wave only, so weights go from the L2 to registers,
@@ -100,9 +101,9 @@ __device__ __forceinline__ void finish_rows(const F32Args& a, const float* ep, i
 // LDS stage: panels [row][64 floats] of 16 chunks of 16 bytes, chunk c of row r in slot
 // c ^ (r & 15): the 16 rows that a quarter-wave reads are 16 different slots.
 // Measured on MI355X (replayed graph; before: both operands through registers into LDS,
-// 32 k ahead): T = 128, hidden 1024, 16 / 8 heads 22.4 -> 16.4 us; T = 256 28.1 -> 23.4;
-// T = 512 44.9 -> 39.8; hidden 2048, 32 / 4 heads T = 300 83.6 -> 71.0; T = 1024
-// 189.7 -> 178.4 (120 TFLOP/s; a large fp32 matrix product reaches 131).
+// 32 k ahead): hidden 1024, 16 / 8 heads T = 256 28.1 -> 23.4 us; T = 512 44.9 -> 39.8;
+// hidden 2048, 32 / 4 heads T = 300 83.6 -> 71.0; T = 1024 189.7 -> 178.4 (120 TFLOP/s; a
+// large fp32 matrix product reaches 131).
 template <int MB>
 struct F32Tile {
   static constexpr int kRows = 16 * MB;
@@ -275,7 +276,7 @@ __device__ __forceinline__ void dma16_from(const void* from, uint32_t off, uint3
 // MFMAs).  So here the weights too go to LDS, as loads of 4 rows x 256 bytes, each wave's
 // 16 columns to a ring of its own that needs no barrier; x comes in units of four stages
 // with one barrier each, and the first reads of a stage are issued under the last MFMAs
-// of the one before.
+// of the one before.  Measured as above: T = 128, hidden 1024, 16 / 8 heads 22.4 -> 16.4 us.
 struct F32Narrow {
   static constexpr int kStageK = 64;
   static constexpr int kPanel = 16 * kStageK;  // floats of 16 rows of one stage (4 KB)

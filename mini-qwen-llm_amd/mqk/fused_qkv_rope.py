@@ -34,8 +34,9 @@ Differences from the reference, all deliberate:
 fp32 inputs (the dtype of the reference's CPU-runnable fp32 layer) take a
 separate kernel: an fp32 projection on the matrix cores (fp32 products and
 sums), norm and RoPE in fp32, fp32 outputs.  fp16 inputs (a model loaded in
-fp16) take the same kernel on the fp16 matrix cores (exact products, fp32
-sums), with fp16 outputs.  Differences from the reference on these dtypes: its
+fp16) take the bf16 kernels on the fp16 matrix cores (exact products, fp32
+sums; a kernel of their own where hidden is no multiple of 64), with fp16
+outputs.  Differences from the reference on these dtypes: its
 Triton kernel rounds Q and K to bf16 before storing them into the fp32 / fp16
 outputs (fused_qkv_rope.py:117-120), and on fp16 its GEMM output is rounded to
 fp16 before the norm; here neither happens, so the outputs carry fp32 / fp16

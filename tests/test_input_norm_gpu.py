@@ -2,8 +2,9 @@
 
 The op must compute the projections of bf16(gamma * bf16(x * rsqrt(mean(x^2) + eps)))
 -- the decoder's input_layernorm (mini_qwen/model/layers/rms_norm.py:15-18, applied
-at qwen3.py:58-59; oracle.rms_norm_hf(..., round_out=True)) -- without writing the
-normalised activations to HBM.
+at qwen3.py:58-59; oracle.rms_norm_hf(..., round_out=True)).  (The package's workspace
+has room for the normalised rows, so these calls write them ahead; the form inside the
+projection kernels is compared with that one in test_norm_ahead_gpu.py.)
 
 * Exactness: V heads whose weight rows are one-hot copy single normalised
   activations through the MFMA unchanged, so ``v`` exposes the kernel's normalised
@@ -94,7 +95,7 @@ def test_input_norm_matches_oracle(B, S, tile, device):
 
 
 def test_input_norm_decode_recompute_path(device):
-    """The split-K decode kernel's recompute path re-stages x and must normalise it again."""
+    """The split-K decode kernel's recompute path re-stages x, which must be the normalised rows."""
     import mqk
     hidden, Hq, Hkv = 1024, 8, 4
     case = Case(1, 16, hidden, Hq, Hkv, seed=700, x_std=2.0)
@@ -147,7 +148,7 @@ def test_input_norm_w4a16(S, tile, device):
 
 
 def test_input_norm_prefill_then_decode_same_workspace(device):
-    """A prefill call with the input norm writes its per-token scales into the
+    """A prefill call with the input norm writes its rows (or per-token scales) into the
     stream's workspace; they must not land on the decode kernel's arrival counters
     (which open the workspace and must stay zero), or a later decode call breaks."""
     import mqk
@@ -166,11 +167,11 @@ def test_input_norm_prefill_then_decode_same_workspace(device):
 
 @pytest.mark.parametrize("T,hidden,plan", [(1536, 8192, ["row_scale", "tile"]), (1536, 4096, ["row_scale", "tile_pair"])])
 def test_input_norm_pair_tiles_need_lds_room(T, hidden, plan, device):
-    """With the input norm, gamma (hidden x 2 bytes) sits in the LDS beside the
-    ring.  At hidden 8192 it does not fit beside the 192-row pair tiles' ring and
-    exchange word (144 KiB + 16 B + 16 KiB), so the planner takes whole-head tiles
-    there; at hidden 4096 the pair tiles run.  Either way the result is the
-    variant-16 launch's, bit for bit."""
+    """Where the tile kernels normalise x themselves, gamma (hidden x 2 bytes) sits in the
+    LDS beside the ring.  At hidden 8192 it does not fit beside the 192-row pair tiles'
+    ring and exchange word (144 KiB + 16 B + 16 KiB), so the planner takes whole-head tiles
+    there, also with the rows written ahead (one plan for both forms); at hidden 4096 the
+    pair tiles run.  Either way the result is the variant-16 launch's, bit for bit."""
     from conftest import launched_kernels
     import mqk
     case = Case(1, T, hidden, 32, 8, seed=5200 + hidden)

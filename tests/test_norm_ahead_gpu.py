@@ -4,12 +4,14 @@ workspace without that room) in the projection kernels.
 Both compute bf16(gamma * bf16(x * scale)) with one scale per token and run the
 same MFMA order wherever they take the same plan, so a call at the C ABI with the
 full workspace and one with the smallest must agree: bit for bit where the launch
-is the same kernel, and within one bf16 ulp where it is not: two differently split
-fp32 sums differ by about 1e-6 of their terms, so their bf16 roundings differ by at
-most one ulp, which is up to 2^-7 of the value (at the foot of a binade); 1e-3 is
-added for values near zero.
+is the same kernel (test_both_forms_agree_on_one_kernel requests it), and within one
+bf16 ulp where it need not be (test_both_forms_agree): two differently split fp32 sums
+differ by about 1e-6 of their terms, so their bf16 roundings differ by at most one ulp,
+which is up to 2^-7 of the value (at the foot of a binade); 1e-3 is added for values
+near zero.  At decode sizes the smallest workspace gets the decode kernel with fewer
+splits and rows ahead, wherever it has more than one.
 Sizes: one token, odd hidden chunk counts (hidden 192: 24 of 64 lanes hold chunks;
-hidden 2112: a partial fifth chunk; 16384: a row of four passes), the block and tile
+hidden 2112: a partial fifth chunk; 16384: a row of two passes), the block and tile
 edges, and int4 weights.
 """
 from __future__ import annotations

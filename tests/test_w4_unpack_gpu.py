@@ -85,6 +85,9 @@ def test_unpacked_weights_are_exact(device):
 
 
 def test_small_calls_keep_the_int4_kernels(device):
+    """The size query makes no room for unpacked weights below the planner's line (nor at
+    hidden 1024).  The line is not the crossover: unpacking would pay for some of the
+    calls just below it."""
     from mqk import _native
     for T, Hq, Hkv, hidden in ((768, 40, 8, 5120), (64, 32, 8, 4096), (8214, 16, 8, 1024)):
         assert _native.fused_workspace_bytes(T, Hq, Hkv, hidden, 128, int4=True) == \
